@@ -193,7 +193,7 @@ def bench_config2(ctx, args):
         step()
     ms = ctx.time_end() / steps
     wall = time.perf_counter() - wall0
-    names = ("xy_fused_kernel", "gemm_f64_xmode", "gemm_f64_ymode", "gemm_f64_zmode",
+    names = ("gemm_f64_xymode", "gemm_f64_xmode", "gemm_f64_ymode", "gemm_f64_zmode",
              "band_xmode", "band_ymode", "band_xymode", "band_zmode", "lowrank",
              "splitk_reduce_kernel",
              "bubbles_inject_kernel", "box_multipoles_kernel", "box_multipoles_gemm",
@@ -208,15 +208,15 @@ def bench_config2(ctx, args):
     ctx.profile(False)
     T = gq.get_npoints()
     # dominant kernel: largest time per step; a GEMM pass does 2 T n^4
-    # dense-equivalent FLOPs per apply, the fused x/y pass twice that (the
+    # dense-equivalent FLOPs per apply, the x/y pass twice that (the
     # zero K panels of the banded near-field matrices are skipped but counted)
     dom = max(kernels, key=lambda k: kernels[k]["ms_per_step"])
     dk = kernels[dom]
-    if dom.startswith("gemm_f64") or dom == "xy_fused_kernel":
-        passes = 2.0 if dom == "xy_fused_kernel" else 1.0
+    if dom.startswith("gemm_f64"):
+        passes = 2.0 if dom == "gemm_f64_xymode" else 1.0
         # the MFMA passes cover the t-points between the low-rank head and the
         # banded tail
-        t_mfma = fmm.band_t0() - fmm.lowrank_t1() if dom.startswith("gemm_f64") else T
+        t_mfma = fmm.band_t0() - fmm.lowrank_t1()
         per_launch = passes * 2.0 * t_mfma * float(n) ** 4 / dk["launches_per_step"]
         achieved = per_launch / (dk["ms_per_launch"] * 1e-3) / 1e12
         roofline = {"bound": "mfma", "kernel": dom, "achieved": round(achieved, 3),
@@ -337,7 +337,7 @@ def bench_config1(ctx, args):
         op.transform_cuda_cube(d_in, d_out)
     ms = ctx.time_end() / steps
     kernels = {}
-    for name in ("xy_fused_kernel", "gemm_f64_xmode", "gemm_f64_ymode", "gemm_f64_zmode",
+    for name in ("gemm_f64_xymode", "gemm_f64_xmode", "gemm_f64_ymode", "gemm_f64_zmode",
                  "band_xmode", "band_ymode", "band_xymode", "band_zmode", "lowrank",
                  "splitk_reduce_kernel"):
         tot, k = ctx.profile_query(name)
@@ -703,11 +703,11 @@ def bench_config5(ctx, args):
     wall = time.perf_counter() - wall0
     # batch_*: the sweep's passes (the batch's own event names); gemm_f64_*:
     # the GBFMM near field's
-    names = ("batch_xy_fused_kernel", "batch_f64_xmode", "batch_f64_ymode", "batch_f64_zmode",
+    names = ("batch_f64_xymode", "batch_f64_xmode", "batch_f64_ymode", "batch_f64_zmode",
              "batch_band_xmode", "batch_band_ymode", "batch_band_xymode", "batch_band_zmode",
              "batch_lowrank",
              "batch_splitk_reduce",
-             "xy_fused_kernel",
+             "gemm_f64_xymode",
              "gemm_f64_xmode", "gemm_f64_ymode", "gemm_f64_zmode", "band_xmode", "band_ymode",
              "band_xymode", "band_zmode", "lowrank",
              "splitk_reduce_kernel",
@@ -736,20 +736,17 @@ def bench_config5(ctx, args):
     T, Tn = hq.get_npoints(), gq.get_npoints()
     # dominant kernel of the step; a mode pass does 2 T n^4 dense FLOPs per
     # right-hand side (sweep: T = 40 for each of 64 orbitals; GBFMM near
-    # field: T = 50 once), the fused x/y pass twice that, counted dense
+    # field: T = 50 once), the x/y pass twice that, counted dense
     # although the all-zero K panels of the banded matrices (exact zeros and
     # the tails stored as zeros below 1e-20 of their row's largest entry) are
     # skipped: `frac` can exceed 1, `frac_executed` counts the executed FLOPs
     dom = max(kernels, key=lambda k: kernels[k]["ms_per_step"])
     dk = kernels[dom]
-    mfma_kernels = ("batch_f64_", "gemm_f64_", "batch_xy_fused", "xy_fused")
-    if dom.startswith(mfma_kernels):
-        passes = 2.0 if "xy_fused" in dom else 1.0
+    if dom.startswith(("batch_f64_", "gemm_f64_")):
+        passes = 2.0 if dom.endswith("xymode") else 1.0
         # the MFMA passes cover the t-points between the low-rank head (applied
         # through factors) and the banded tail (VALU passes)
-        if "xy_fused" in dom:
-            tsum = T * nrhs if dom.startswith("batch_") else Tn
-        elif dom.startswith("batch_"):
+        if dom.startswith("batch_"):
             probe = dage_amd.Helmholtz3D(ctx, grid, grid, hq)
             til = probe.tiling()
             tsum = (til["band_t0"] - til["lowrank_t1"]) * nrhs
@@ -764,7 +761,7 @@ def bench_config5(ctx, args):
                     "frac": round(achieved / FP64_MFMA_PEAK_TFLOPS, 4),
                     "traffic": measured_traffic("config5", dom),
                     "flops": "dense-equivalent (2 T n^4 per pass and right-hand side; the "
-                             "fused x/y kernel does two passes); the skipped all-zero panels "
+                             "x/y kernel does two passes); the skipped all-zero panels "
                              "count, so frac can exceed 1: frac_executed is the MFMA use",
                     "avg_launch_ms": dk["ms_per_launch"],
                     "launches_per_step": dk["launches_per_step"],

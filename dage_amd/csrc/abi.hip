@@ -185,10 +185,12 @@ void free_operator_buffers(dage_operator op) {
     op->d_mask = nullptr;
     if (op->d_tmask) (void)hipFree(op->d_tmask);
     op->d_tmask = nullptr;
-    if (op->d_xband) (void)hipFree(op->d_xband);
-    op->d_xband = nullptr;
-    if (op->d_yband) (void)hipFree(op->d_yband);
-    op->d_yband = nullptr;
+    if (op->d_ranges) (void)hipFree(op->d_ranges);
+    op->d_ranges = nullptr;
+    if (op->d_steps) (void)hipFree(op->d_steps);
+    op->d_steps = nullptr;
+    if (op->d_pack) (void)hipFree(op->d_pack);
+    op->d_pack = nullptr;
     if (op->d_band) (void)hipFree(op->d_band);
     op->d_band = nullptr;
     if (op->d_lr) (void)hipFree(op->d_lr);
@@ -243,8 +245,7 @@ int dage_ctx_create(int device, dage_ctx *out) {
         return DAGE_ERR_HIP;
     }
     ctx->stream = ctx->own_stream;
-    int rc = prepare_fused_kernels();
-    if (rc == DAGE_OK) rc = scratch_address(device, &ctx->noalloc_scratch);
+    const int rc = scratch_address(device, &ctx->noalloc_scratch);
     if (rc != DAGE_OK) {
         (void)hipStreamDestroy(ctx->own_stream);
         delete ctx;

@@ -388,176 +388,6 @@ __global__ void __launch_bounds__(kThreads) gemm_f64_kernel(Gemm g) {
     }
 }
 
-// Fused x and y passes: for one (right-hand side b, t, input z-plane zi) and
-// 64 output x points (16 per wavefront),
-//   U(xo, yo) = w_t sum_yi [sum_xi Fx_t(xo,xi) in(xi,yi,zi)] Fy_t(yi,yo),
-// without the x-pass intermediate V reaching memory.  The input y axis is
-// walked in chunks of 16 points.  Per chunk a wavefront first forms the
-// 16 x 16 tile V^T(yi, xo) = in^T(yi, xi) Fx_t^T(xi, xo) on the MFMA (A = the
-// input chunk from LDS, B = Fx_t from global memory); result register r of
-// lane l then holds V(xo = l%16, yi = 4r + l/16), which is exactly the
-// A-operand element of k-step r of the y product, so the tile feeds
-//   U(xo, yo) += V(xo, yi-chunk) Fy_t(yi-chunk, yo)
-// straight from registers (B = the Fy_t chunk from LDS), one accumulator per
-// 16-point output y tile.  The k-grouping, operand roles and k order are those
-// of the separate x and y passes, and only products with a zero matrix entry
-// outside the bands are skipped, so U is bit-identical to theirs.
-//
-// The input chunk (16 columns of nxi points, contiguous in memory) and the
-// Fy_t chunk (16 rows) are staged in LDS, the next chunk's loads issued into
-// registers before the current chunk's MFMAs.  NT >= the output y tiles and
-// NT >= nxi / 16 (it also sizes the loader's registers).
-struct XYF {
-    const double *in;   // in_b(xi, yi, zi) at in + b*nin + xi + nxi*(yi + nyi*zi)
-    const double *fx;   // Fx_t(xo, xi) at fx + xo + nxo*(xi + nxi*t)
-    const double *fy;   // Fy_t(yi, yo) at fy + yi + nyi*(yo + nyo*t)
-    double *U;          // U + xo + nxo*(yo + nyo*zi) + Ut*(tl + tc*b)
-    const double *w;    // alpha = w[t0 + tl + wS*b]
-    long wS;
-    int nxi, nyi, nxo, nyo, nzi;
-    int t0, tc;
-    long nin, Ut;
-    const int2 *xband, *yband;
-    int nxt, nyc;
-    int gx;      // 64-point output x blocks
-    int ldy;     // LDS row count of the Fy chunk (16 * output y tiles)
-    int remap;
-};
-
-template <int NT>
-__global__ void __launch_bounds__(kThreads) xy_fused_kernel(XYF g) {
-    extern __shared__ double smem[];
-    double *Is = smem;                   // input chunk: (xi, yl) at yl*nxi + xi
-    double *Ys = smem + 16 * g.nxi;      // Fy chunk: (yl, yo) at yo*17 + yl
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int l16 = lane & 15, lk = lane >> 4;
-
-    // block -> (b, tl, zi, xb), xb fastest; XCD-aware as in block_coords
-    unsigned L = blockIdx.x;
-    if (g.remap) {
-        const unsigned total = gridDim.x;
-        const unsigned q = total >> 3, r = total & 7u, x = L & 7u;
-        L = x * q + min(x, r) + (L >> 3);
-    }
-    const int xb = (int)(L % (unsigned)g.gx);
-    L /= (unsigned)g.gx;
-    const int zi = (int)(L % (unsigned)g.nzi);
-    L /= (unsigned)g.nzi;
-    const int tl = (int)(L % (unsigned)g.tc);
-    const int b = (int)(L / (unsigned)g.tc);
-    const int t = g.t0 + tl;
-
-    const double *in = g.in + (long)b * g.nin + (long)zi * g.nxi * g.nyi;
-    const double *fx = g.fx + (long)t * g.nxo * g.nxi;
-    const double *fy = g.fy + (long)t * g.nyi * g.nyo;
-    const int xt = xb * 4 + wave;  // this wavefront's 16-point output x tile
-    const bool active = xt < g.nxt;
-    const int xo = xt * 16 + l16;
-    const bool xo_ok = xo < g.nxo;
-    const int2 xr = active ? g.xband[(long)t * g.nxt + xt] : make_int2(0, 0);
-    const double *fxl = fx + (xo_ok ? xo : 0);
-
-    // loaders: input chunk element e = tid + 256*s (contiguous in memory),
-    // Fy chunk element e: yl = e % 16, yo = e / 16
-    const int ichunk = 16 * g.nxi;
-    double ri[NT], ry[NT];
-    auto load_chunk = [&](int c) {
-        const int yc = 16 * c;
-        const int ilim = min(16, g.nyi - yc) * g.nxi;  // valid elements
-        const double *src = in + (long)yc * g.nxi;
-#pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            const int e = tid + kThreads * s;
-            const bool ok = e < ilim;
-            const double v = src[ok ? e : 0];
-            ri[s] = ok ? v : 0.0;
-        }
-#pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            const int e = tid + kThreads * s;
-            const int yl = e & 15, yo = e >> 4;
-            const bool ok = yo < g.nyo && yc + yl < g.nyi;
-            const double v = fy[ok ? (long)(yc + yl) + (long)g.nyi * yo : 0];
-            ry[s] = ok ? v : 0.0;
-        }
-    };
-    auto store_chunk = [&]() {
-#pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            const int e = tid + kThreads * s;
-            if (e < ichunk) Is[e] = ri[s];
-        }
-#pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            const int e = tid + kThreads * s;
-            const int yl = e & 15, yo = e >> 4;
-            if (yo < g.ldy) Ys[yo * 17 + yl] = ry[s];
-        }
-    };
-
-    d4 acc[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[j] = d4{0.0, 0.0, 0.0, 0.0};
-
-    const int nchunks = (g.nyi + 15) / 16;
-    load_chunk(0);
-    for (int c = 0; c < nchunks; ++c) {
-        store_chunk();
-        __syncthreads();
-        if (c + 1 < nchunks) load_chunk(c + 1);
-        const int2 yr = g.yband[(long)t * g.nyc + c];
-        if (active && yr.x < yr.y && xr.x < xr.y) {
-            // x part: V^T(yi, xo) over the k-steps of this tile's band
-            d4 v = d4{0.0, 0.0, 0.0, 0.0};
-            const double *ia = Is + l16 * g.nxi;
-            for (int s0 = xr.x; s0 < xr.y; s0 += 8) {
-                double fa[8], fb[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int xi = 4 * (s0 + u) + lk;
-                    const bool ok = s0 + u < xr.y && xi < g.nxi;
-                    const double bv = fxl[ok && xo_ok ? (long)g.nxo * xi : 0];
-                    fb[u] = ok && xo_ok ? bv : 0.0;
-                    fa[u] = ok ? ia[ok ? xi : 0] : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (s0 + u < xr.y) v = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u], fb[u], v, 0, 0, 0);
-            }
-            // y part: k-steps with some input y point inside the grid
-            const int nks = min(4, (g.nyi - 16 * c + 3) / 4);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                if (s < nks) {
-#pragma unroll
-                    for (int j = 0; j < NT; ++j)
-                        if (j >= yr.x && j < yr.y) {
-                            const double bv = Ys[(16 * j + l16) * 17 + 4 * s + lk];
-                            acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s], bv, acc[j], 0, 0, 0);
-                        }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    if (!active) return;
-    // Register r of lane l holds U(xo = xt*16 + 4r + l/16, yo = 16j + l%16).
-    const double alpha = g.w[g.t0 + tl + g.wS * b];
-    double *U = g.U + (long)zi * g.nxo * g.nyo + g.Ut * ((long)tl + (long)g.tc * b);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const int yo = 16 * j + l16;
-        if (yo >= g.nyo) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int x = xt * 16 + 4 * r + lk;
-            if (x < g.nxo) U[x + (long)g.nxo * yo] = alpha * acc[j][r];
-        }
-    }
-}
-
 // Fz (nzi, nzo, T) -> Gz((zi + nzi*t), zo)
 __global__ void __launch_bounds__(256) relayout_fz_kernel(const double *fz, double *gz, int nzi,
                                                           int nzo, int T) {
@@ -710,15 +540,6 @@ int launch_gemm(dage_ctx ctx, const char *name, const Gemm &g, int zdim, int nb_
     return rc;
 }
 
-// Fused x/y pass (xy_fused_kernel): opt-in with DAGE_APPLY_FUSED=1, when the
-// bands are built and both the output y axis and the input x axis fit the
-// largest register tile.  Measured on MI355X it is 1.5x (97^3) to 4.4x
-// (385^3) slower than the separate x and y passes: per chunk each wavefront's
-// x product is one dependent MFMA chain fed by global loads of Fx_t, at one
-// wavefront per SIMD once the y accumulators pass 128 registers.  Returns
-// the kernel's NT (0: separate passes).
-constexpr int kMaxNT = 28;
-
 // The x pass with 4 t-points per block (PASS 4) where the cost model picks
 // 16- or 32-column tiles; DAGE_APPLY_TGROUP=0 keeps one t per block.
 // Measured on the 385^3 sweep's middle t-points: 23.6 ms per launch against
@@ -729,76 +550,29 @@ bool tgroup_x() {
     return !(e && e[0] == '0');
 }
 
-int fused_nt(const ApplyMats &m) {
-    if (!m.xband || !m.yband) return 0;
-    const char *e = std::getenv("DAGE_APPLY_FUSED");
-    if (!e || e[0] != '1') return 0;
-    const int need = std::max((m.dout[1] + 15) / 16, (m.din[0] + 15) / 16);
-    if (need > kMaxNT) return 0;
-    return (need + 3) / 4 * 4;
-}
-
-// Largest dynamic LDS of the fused pass: 16 input columns of up to 16*kMaxNT
-// points and 16*kMaxNT Fy rows of 17 doubles.
-constexpr size_t kFusedMaxLds = 8 * (16 * 16 * kMaxNT + 17 * 16 * kMaxNT);
-
-template <int NT>
-int set_xy_attr() {
-    DAGE_HIP_CHECK(hipFuncSetAttribute((const void *)xy_fused_kernel<NT>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)kFusedMaxLds));
-    return DAGE_OK;
-}
-
-template <int NT>
-int launch_xy_t(const XYF &g, unsigned blocks, size_t lds, hipStream_t s) {
-    hipLaunchKernelGGL(xy_fused_kernel<NT>, dim3(blocks), dim3(kThreads), lds, s, g);
-    DAGE_HIP_CHECK(hipGetLastError());
-    return DAGE_OK;
-}
-
-int launch_xy(dage_ctx ctx, int nt, const XYF &g, int B, const char *name) {
-    const long blocks = (long)g.gx * g.nzi * g.tc * B;
-    DAGE_REQUIRE(blocks > 0 && blocks < (1L << 31), DAGE_ERR_ARG,
-                 "fused pass of %ld blocks does not fit one launch", blocks);
-    DAGE_REQUIRE(16 * nt >= g.ldy && 16 * nt >= g.nxi, DAGE_ERR_STATE,
-                 "fused pass tile %d too small", nt);
-    const size_t lds = 8 * (16 * (size_t)g.nxi + 17 * (size_t)g.ldy);
-    hipEvent_t ev;
-    prof_begin(ctx, name, &ev);
-    int rc;
-    const unsigned nb = (unsigned)blocks;
-    switch (nt) {
-    case 4: rc = launch_xy_t<4>(g, nb, lds, ctx->stream); break;
-    case 8: rc = launch_xy_t<8>(g, nb, lds, ctx->stream); break;
-    case 12: rc = launch_xy_t<12>(g, nb, lds, ctx->stream); break;
-    case 16: rc = launch_xy_t<16>(g, nb, lds, ctx->stream); break;
-    case 20: rc = launch_xy_t<20>(g, nb, lds, ctx->stream); break;
-    case 24: rc = launch_xy_t<24>(g, nb, lds, ctx->stream); break;
-    case 28: rc = launch_xy_t<28>(g, nb, lds, ctx->stream); break;
-    default: DAGE_REQUIRE(false, DAGE_ERR_STATE, "no fused pass for tile %d", nt);
-    }
-    prof_end(ctx, name, ev);
-    return rc;
-}
-
-// Workspace layout: V | U | P (split-K partials); no V with the fused pass
+// Workspace layout: V | U | P (split-K partials); the streamed passes, which
+// have no V, use V | U as one U.  DAGE_APPLY_FUSED=1 plans without V (and
+// without the banded and low-rank t-points) where every t-point streams:
+// half the workspace at one t-point, so larger cubes fit a limited scratch.
 struct Plan {
     int tchunk;
     int splits;
+    bool no_v;
     size_t v_elems, u_elems, p_elems;
 };
 
 // cap > 0: the whole workspace must fit cap bytes (the largest t-chunk, then
 // the largest K split, that does); tchunk = 0 when nothing fits.
 Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
-    const bool fused = fused_nt(m) > 0;
     const long nyi = m.din[1], nzi = m.din[2];
     const long nxo = m.dout[0], nyo = m.dout[1], nzo = m.dout[2];
     size_t budget = 4ull << 30;  // bytes for V + U per right-hand side
     if (const char *e = std::getenv("DAGE_APPLY_WORKSPACE_MB")) budget = (size_t)atol(e) << 20;
     const size_t total_cap = 64ull << 30;  // and for all B right-hand sides together
-    const size_t per_t = 8ull * (size_t)((fused ? 0 : nxo * nyi * nzi) + nxo * nyo * nzi);
+    const char *fu = std::getenv("DAGE_APPLY_FUSED");
+    const bool no_v = fu && fu[0] == '1' && streams_all(m);
+    const size_t vt = no_v ? 0 : (size_t)(nxo * nyi * nzi);
+    const size_t per_t = 8ull * (vt + (size_t)(nxo * nyo * nzi));
     const long M3 = nxo * nyo;
     const int mtiles = (int)((M3 + 64 * kMW - 1) / (64 * kMW));
     const int nb = pick_nb((int)nzo);
@@ -806,11 +580,13 @@ Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
     auto fill = [&](int tchunk) {
         Plan p;
         p.tchunk = tchunk;
+        p.no_v = no_v;
         const long K3 = nzi * p.tchunk;
-        int splits = std::max(1, (1024 + mtiles * ntiles * B - 1) / (mtiles * ntiles * B));
+        int splits = m.fxp ? z_splits(m, B)
+                           : std::max(1, (1024 + mtiles * ntiles * B - 1) / (mtiles * ntiles * B));
         splits = (int)std::min<long>(splits, std::max<long>(1, K3 / 64));
         p.splits = splits;
-        p.v_elems = fused ? 0 : (size_t)nxo * nyi * nzi * p.tchunk * B;
+        p.v_elems = vt * p.tchunk * B;
         p.u_elems = (size_t)nxo * nyo * nzi * p.tchunk * B;
         p.p_elems = (size_t)M3 * nzo * splits * B;
         return p;
@@ -832,17 +608,16 @@ Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
         none.tchunk = 0;
         return none;
     }
-    // DAGE_APPLY_TCHUNK: a fixed t-chunk (comparison runs; the z pass then adds
-    // the same partial sums in the same order with or without the fused pass)
+    // DAGE_APPLY_TCHUNK: a fixed t-chunk (comparison runs)
     if (const char *e = std::getenv("DAGE_APPLY_TCHUNK"))
         if (atoi(e) > 0) return fill(std::min(m.ntp, atoi(e)));
     return fill((int)std::max<size_t>(
         1, std::min<size_t>({(size_t)m.ntp, budget / per_t, total_cap / (per_t * (size_t)B)})));
 }
 
-// out[b*len + i] = sum_s part[(b*splits + s)*len + i] + coda*in[b*len + i]
+// out[b*len + i] = sum_{s < splits} part[(b*stride + s)*len + i] + coda*in[b*len + i]
 __global__ void __launch_bounds__(256) splitk_reduce_batch_kernel(const double *part, int splits,
-                                                                  long len, int B,
+                                                                  int stride, long len, int B,
                                                                   const double *in, double coda,
                                                                   double *out) {
     const long total = len * B;
@@ -850,7 +625,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_batch_kernel(const double *
          e += (long)gridDim.x * blockDim.x) {
         const long b = e / len, i = e - b * len;
         double s = 0.0;
-        for (int k = 0; k < splits; ++k) s += part[(b * splits + k) * len + i];
+        for (int k = 0; k < splits; ++k) s += part[(b * stride + k) * len + i];
         if (in) s += coda * in[e];
         out[e] = s;
     }
@@ -1118,50 +893,7 @@ int build_masks(dage_operator op) {
         }
     }
     DAGE_HIP_CHECK(hipMemcpyAsync(op->d_tmask, ht.data(), 8 * ht.size(), hipMemcpyHostToDevice, s));
-    // Bands of the fused x/y pass from the row spans: output x tile j (16
-    // points) takes input points xi whose Fx_t row reaches it, input y chunk
-    // c (16 points) reaches the output y tiles its Fy_t rows span.  Zero
-    // entries inside a band are computed (they add exact zeros).
-    const int nxt = (int)((nxo + 15) / 16), nyc = (int)((nyi + 15) / 16);
-    std::vector<int2> xb((size_t)T * nxt), yb((size_t)T * nyc);
-    for (long t = 0; t < T; ++t) {
-        for (int j = 0; j < nxt; ++j) {
-            const int a = 16 * j, b = (int)std::min<long>(a + 16, nxo);
-            long lo = -1, hi = -1;
-            for (long xi = 0; xi < nxi; ++xi) {
-                const long r = t * nxi + xi;
-                if (hs[2 * r] < b && hs[2 * r + 1] >= a) {
-                    if (lo < 0) lo = xi;
-                    hi = xi;
-                }
-            }
-            xb[t * nxt + j] = lo < 0 ? make_int2(0, 0) : make_int2((int)(lo / 4), (int)(hi / 4 + 1));
-        }
-        for (int c = 0; c < nyc; ++c) {
-            int lo = 1 << 30, hi = -1;
-            for (long yi = 16L * c; yi < std::min<long>(16L * c + 16, nyi); ++yi) {
-                const long r = rx + t * nyi + yi;
-                if (hs[2 * r + 1] >= 0) {
-                    lo = std::min(lo, hs[2 * r] / 16);
-                    hi = std::max(hi, hs[2 * r + 1] / 16);
-                }
-            }
-            yb[t * nyc + c] = hi < 0 ? make_int2(0, 0) : make_int2(lo, hi + 1);
-        }
-    }
-    if (op->nxt != nxt || op->nyc != nyc || !op->d_xband) {
-        if (op->d_xband) DAGE_HIP_CHECK(hipFree(op->d_xband));
-        if (op->d_yband) DAGE_HIP_CHECK(hipFree(op->d_yband));
-        op->d_xband = op->d_yband = nullptr;
-        DAGE_HIP_CHECK(hipMalloc((void **)&op->d_xband, sizeof(int2) * xb.size()));
-        DAGE_HIP_CHECK(hipMalloc((void **)&op->d_yband, sizeof(int2) * yb.size()));
-        op->nxt = nxt;
-        op->nyc = nyc;
-    }
-    DAGE_HIP_CHECK(hipMemcpyAsync(op->d_xband, xb.data(), sizeof(int2) * xb.size(),
-                                  hipMemcpyHostToDevice, s));
-    DAGE_HIP_CHECK(hipMemcpyAsync(op->d_yband, yb.data(), sizeof(int2) * yb.size(),
-                                  hipMemcpyHostToDevice, s));
+    DAGE_TRY(build_stream(op, hs));
     DAGE_HIP_CHECK(hipStreamSynchronize(s));
     // tuning knob "x,y,z": fixed column-block counts, masks on wherever defined
     if (const char *e = std::getenv("DAGE_APPLY_NB")) {
@@ -1188,10 +920,7 @@ ApplyMats operator_mats(dage_operator op) {
         m.dout[i] = op->dout[i];
     }
     m.ntp = op->ntp;
-    m.xband = op->d_xband;
-    m.yband = op->d_yband;
-    m.nxt = op->nxt;
-    m.nyc = op->nyc;
+    stream_mats(op, &m);
     m.band_t0 = op->ntp;
     if (op->d_band) {
         m.band_t0 = op->band_t0;
@@ -1216,17 +945,6 @@ ApplyMats operator_mats(dage_operator op) {
         }
     }
     return m;
-}
-
-int prepare_fused_kernels() {
-    DAGE_TRY(set_xy_attr<4>());
-    DAGE_TRY(set_xy_attr<8>());
-    DAGE_TRY(set_xy_attr<12>());
-    DAGE_TRY(set_xy_attr<16>());
-    DAGE_TRY(set_xy_attr<20>());
-    DAGE_TRY(set_xy_attr<24>());
-    DAGE_TRY(set_xy_attr<28>());
-    return DAGE_OK;
 }
 
 int apply_f64_workspace(dage_operator op, size_t *bytes) {
@@ -1289,11 +1007,10 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
     // which later t-chunks still read.
     const bool direct = B == 1 && plan.splits == 1 && bs.coda == 0.0 &&
                         (out + nout <= in || in + nin <= out);
-    const int nt = fused_nt(m);
     // event names (profiling): batched right-hand sides with their own
     // weights (the batch graph) apart from single applies
     const bool bat = bs.w != nullptr;
-    const char *nm_xy = bat ? "batch_xy_fused_kernel" : "xy_fused_kernel";
+    const char *nm_xy = bat ? "batch_f64_xymode" : "gemm_f64_xymode";
     const char *nm_x = bat ? "batch_f64_xmode" : "gemm_f64_xmode";
     const char *nm_y = bat ? "batch_f64_ymode" : "gemm_f64_ymode";
     const char *nm_z = bat ? "batch_f64_zmode" : "gemm_f64_zmode";
@@ -1302,50 +1019,51 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
     const char *nm_bxy = bat ? "batch_band_xymode" : "band_xymode";
     const char *nm_by = bat ? "batch_band_ymode" : "band_ymode";
     const char *nm_bz = bat ? "batch_band_zmode" : "band_zmode";
+    const long slab = M3 * nzo;
+    // partials (per right-hand side) that hold a sum already; the first pass
+    // that writes one overwrites it
+    int pinit = 0;
     // t-points from tb on (narrow bands) take the banded passes; the MFMA
     // chunks stop there
-    const int tb = (nt == 0 && band_pays(m, B)) ? m.band_t0 : T;
+    const int tb = !plan.no_v && band_pays(m, B) ? m.band_t0 : T;
     // the low-rank t-points (the smallest t) first, when their intermediates
-    // fit the passes' workspace: partial 0 (or out) is overwritten, the other
-    // partials cleared, and the chunks below accumulate
+    // fit the passes' workspace, into partial 0 (or out)
     int tlr = 0;
-    if (nt == 0 && lowrank_pays(m, B)) {
+    if (!plan.no_v && lowrank_pays(m, B)) {
         size_t w1 = 0, w2 = 0;
         lowrank_workspace(m, B, &w1, &w2);
         if (w1 <= plan.v_elems && w2 <= plan.u_elems) {
-            const long slab = M3 * nzo;
-            if (!direct)
-                for (int b = 0; b < B && plan.splits > 1; ++b)
-                    DAGE_TRY(fill_zero(ctx, P + ((size_t)b * plan.splits + 1) * slab,
-                                       (size_t)(plan.splits - 1) * slab));
             DAGE_TRY(lowrank_apply(ctx, m, in, direct ? out : P, (long)plan.splits * slab, B, W,
                                    wS, V, U, bat ? "batch_lowrank" : "lowrank"));
             tlr = m.lr->t1;
+            pinit = 1;
         }
     }
+    // t-points whose U the streamed passes can hold at once in V | U
+    const int tstream = std::getenv("DAGE_APPLY_TCHUNK")
+                            ? tcmax : (int)((plan.v_elems + plan.u_elems) / ((size_t)Ut * B));
     for (int t0 = tlr; t0 < T;) {
         const bool banded = t0 >= tb;
-        const int tc = std::min(tcmax, (banded ? T : tb) - t0);
-        if (nt > 0) {
-            // passes 1 and 2 fused: U_b((xo,yo),(zi,t)) straight from in_b
-            XYF f{};
-            f.in = in;
-            f.fx = m.fx;
-            f.fy = m.fy;
-            f.U = U;
-            f.w = W;
-            f.wS = wS;
-            f.nxi = (int)nxi; f.nyi = (int)nyi; f.nxo = (int)nxo; f.nyo = (int)nyo;
-            f.nzi = (int)nzi;
-            f.t0 = t0; f.tc = tc;
-            f.nin = nin; f.Ut = Ut;
-            f.xband = m.xband; f.yband = m.yband;
-            f.nxt = m.nxt; f.nyc = m.nyc;
-            f.gx = (int)((nxo + 63) / 64);
-            f.ldy = 16 * (int)((nyo + 15) / 16);
-            f.remap = remap_default(8.0 * nxi * nyi * nzi);
-            DAGE_TRY(launch_xy(ctx, nt, f, B, nm_xy));
-        } else {
+        if (!banded) {
+            const int tend = std::min(tb, t0 + tstream);
+            int tc = 0, tiles = 0;
+            while (const int r = stream_run(m, t0 + tc, tend, B, &tiles)) {
+                DAGE_TRY(stream_xy(ctx, m, tiles, in, V, Ut, Ut * tstream, t0, W, wS, t0 + tc, r, B, nm_xy));
+                tc += r;
+            }
+            if (tc > 0) {
+                const int splits = plan.splits;
+                DAGE_TRY(stream_z(ctx, m, V, Ut, Ut * tstream, t0, direct ? out : P,
+                                  slab * plan.splits, slab, splits, pinit, t0, tc, B, nm_z));
+                pinit = std::max(pinit, splits);
+                t0 += tc;
+                continue;
+            }
+        }
+        int tc = std::min(tcmax, (banded ? T : tb) - t0), tiles = 0;
+        if (!banded)  // up to the next t-point that can be streamed
+            for (int e = 1; e < tc; ++e)
+                if (stream_run(m, t0 + e, t0 + e + 1, B, &tiles) > 0) tc = e;
         // pass 1, batch (t, b): V_{b,t}((yi,zi), xo) = in_b((yi,zi), xi) . Fx_t^T(xi, xo)
         Gemm g1{};
         g1.A = in;
@@ -1399,18 +1117,12 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
         set_tiles(g2, 1, (long)t0 * nyi, nyi, &nb2);
         DAGE_TRY(launch_gemm<1>(ctx, nm_y, g2, tc * B, nb2));
         }
-        }
 
         if (banded) {
-            // into partial 0 of each right-hand side (the others are zero when
-            // no MFMA chunk ran before), or straight into out
-            const long slab = M3 * nzo;
-            if (t0 == 0 && !direct)
-                for (int b = 0; b < B && plan.splits > 1; ++b)
-                    DAGE_TRY(fill_zero(ctx, P + ((size_t)b * plan.splits + 1) * slab,
-                                       (size_t)(plan.splits - 1) * slab));
-            DAGE_TRY(band_pass_z(ctx, m, U, direct ? out : P, (long)plan.splits * slab, t0 > 0,
+            // into partial 0 of each right-hand side, or straight into out
+            DAGE_TRY(band_pass_z(ctx, m, U, direct ? out : P, (long)plan.splits * slab, pinit > 0,
                                  t0, tc, B, nm_bz));
+            pinit = std::max(pinit, 1);
             t0 += tc;
             continue;
         }
@@ -1430,24 +1142,25 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
         g3.bC = M3 * nzo;
         g3.Z0 = splits; g3.bA1 = Ut * tc; g3.bB1 = 0; g3.bC1 = M3 * nzo * plan.splits;
         g3.Ksplit = ks;
-        g3.accumulate = (t0 > 0);
+        g3.accumulate = pinit > 0;
         int nb3;
         set_tiles(g3, 2, (long)nzi * t0, 0, &nb3);
-        if (t0 == 0 && splits < plan.splits)
+        if (pinit > 0 && pinit < splits)
             for (int b = 0; b < B; ++b)
-                DAGE_TRY(fill_zero(ctx, P + ((size_t)b * plan.splits + splits) * M3 * nzo,
-                                   (size_t)(plan.splits - splits) * M3 * nzo));
+                DAGE_TRY(fill_zero(ctx, P + ((size_t)b * plan.splits + pinit) * slab,
+                                   (size_t)(splits - pinit) * slab));
         DAGE_TRY(launch_gemm<2>(ctx, nm_z, g3, splits * B, nb3));
+        pinit = std::max(pinit, splits);
         t0 += tc;
     }
     if (direct) return DAGE_OK;
-    const long len = M3 * nzo;
+    const long len = slab;
     const long total = len * B;
     const int grid = (int)std::min<long>((total + 255) / 256, 65536);
     hipEvent_t ev;
     prof_begin(ctx, nm_r, &ev);
     hipLaunchKernelGGL(splitk_reduce_batch_kernel, dim3(grid), dim3(256), 0, ctx->stream, P,
-                       plan.splits, len, B, bs.coda != 0.0 ? in : nullptr, bs.coda, out);
+                       pinit, plan.splits, len, B, bs.coda != 0.0 ? in : nullptr, bs.coda, out);
     DAGE_HIP_CHECK(hipGetLastError());
     prof_end(ctx, nm_r, ev);
     return DAGE_OK;
@@ -1475,7 +1188,7 @@ int gemm_colmajor(dage_ctx ctx, const char *name, int M, int N, int K, const dou
     const long len = (long)M * N;
     const int grid = (int)std::min<long>((len + 255) / 256, 65536);
     hipLaunchKernelGGL(splitk_reduce_batch_kernel, dim3(grid), dim3(256), 0, ctx->stream, part,
-                       nsplit, len, 1, (const double *)nullptr, 0.0, C);
+                       nsplit, nsplit, len, 1, (const double *)nullptr, 0.0, C);
     DAGE_HIP_CHECK(hipGetLastError());
     return DAGE_OK;
 }

@@ -235,12 +235,19 @@ struct dage_operator_s {
     // banded tail); mix_pitch[p] is 0 or pitch[p]
     int mix_nb_pick[3] = {0, 0, 0}, mix_pitch[3] = {0, 0, 0}, mix_nbp[3] = {0, 0, 0};
     bool mix_mask_used[3] = {false, false, false};
-    // Nonzero bands for the fused x/y pass: d_xband[t*nxt + j] = [first,
-    // last+1) k-step (4 input x points) of Fx_t rows reaching output x tile j
-    // (16 points); d_yband[t*nyc + c] = [first, last+1) 16-point output y tile
-    // reached by Fy_t rows of input y chunk c (16 points)
-    int2 *d_xband = nullptr, *d_yband = nullptr;
-    int nxt = 0, nyc = 0;
+    // Streamed passes (stream.hip): d_ranges holds per t and 16-point output
+    // tile the range [first, last+1) of k-steps (4 input points) whose rows
+    // reach the tile (x, y, z tiles); d_pack the
+    // matrices in MFMA fragment blocks, x, y, z at pack_off; tile_hb[t] the
+    // tiles to either side of the diagonal that hold every x and y range
+    int2 *d_ranges = nullptr;
+    double *d_pack = nullptr;
+    size_t pack_off[3] = {0, 0, 0};
+    std::vector<int> tile_hb;
+    // d_steps: the z pass's lists of panels, for each group of output tiles,
+    // each number of splits S and split s of it from z_off[.] on; z_t: their t
+    int4 *d_steps = nullptr;
+    std::vector<int> z_off, z_t;
     void *d_planes = nullptr;   // split-BF16 matrix planes (built on first mixed apply)
     bool planes_valid = false;  // cleared when the matrices change
     MixedLayout mixed;
@@ -298,9 +305,11 @@ struct ApplyMats {
     // pitch tiling (pitch[p] > 0): tile masks, same row order, bit j = tile j
     const uint64_t *tmask[3] = {nullptr, nullptr, nullptr};
     int pitch[3] = {0, 0, 0}, nbp[3] = {0, 0, 0};
-    // nonzero bands of Fx and Fy (dage_operator_s::d_xband/d_yband; null: none)
-    const int2 *xband = nullptr, *yband = nullptr;
-    int nxt = 0, nyc = 0;
+    // streamed passes (dage_operator_s::d_pack, d_ranges, tile_hb; null: none)
+    const double *fxp = nullptr, *fyp = nullptr, *fzp = nullptr;
+    const int2 *xr = nullptr, *yr = nullptr;
+    const int *hb = nullptr, *z_off = nullptr, *z_t = nullptr;
+    const int4 *zsteps = nullptr;
     // banded y/z passes for t >= band_t0 (see dage_operator_s)
     const double *band_y = nullptr, *band_z = nullptr, *band_x = nullptr;
     int band_t0 = 0, band_mode = 1;
@@ -334,9 +343,6 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
                     const BatchSpec &bs, Workspace *ws);
 int apply_f64_batch_workspace(const ApplyMats &m, int B, size_t *bytes);
 int apply_f64_workspace(dage_operator op, size_t *bytes);
-// Allows the fused x/y pass its dynamic LDS on the current device (called
-// once per context, outside any stream capture).
-int prepare_fused_kernels();
 // Mixed-precision apply (apply_mixed.hip): npair = 6 (bf16x6) or 3 (bf16x3).
 int apply_mixed(dage_operator op, const double *in_dev, double *out_dev, int npair);
 // Batch of right-hand sides on one operator (same conventions as apply_f64_batch).
@@ -411,6 +417,25 @@ int flush_matrices(dage_operator op);
 // C (+)= sum_t U_t . Fz_t over t = t0..t0+tc-1 (all >= band_t0), for B
 // right-hand sides, in the layouts of apply_f64.hip's passes 2 and 3.
 int build_bands(dage_operator op, const std::vector<int> &span);
+// Streamed MFMA passes (stream.hip).  tile_ranges: the k-step ranges of one
+// axis at one t from its rows' spans; returns their half-width in tiles.
+int tile_ranges(const int *span, long row0, long n, long no, int2 *out);
+// Packed matrices and tables (from build_masks, with its row spans), and
+// their pointers for an apply.
+int build_stream(dage_operator op, const std::vector<int> &span);
+void stream_mats(dage_operator op, ApplyMats *m);
+// Number of leading t-points of [t0, t1) one stream_xy call of B right-hand
+// sides takes (0: t0 cannot be streamed) and its kernel's tiles.
+int stream_run(const ApplyMats &m, int t0, int t1, int B, int *tiles);
+bool streams_all(const ApplyMats &m);
+int z_splits(const ApplyMats &m, int B);
+// U_{b,t} (at U + b*Ub + (t - tu)*Ut) = w_{b,t} (x and y products of in_b)
+int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, double *U, long Ut,
+              long Ub, int tu, const double *w, long wS, int t0, int tc, int B, const char *name);
+// Partial s < splits of b (C + b*cB + s*cS): its part of the z products of
+// t0..t0+tc-1; partials below ninit accumulate, the others are overwritten
+int stream_z(dage_ctx ctx, const ApplyMats &m, const double *U, long Ut, long Ub, int tu, double *C,
+             long cB, long cS, int splits, int ninit, int t0, int tc, int B, const char *name);
 // Whether an apply of B right-hand sides takes the banded passes.
 bool band_pays(const ApplyMats &m, int B);
 // Column-major FP64 MFMA GEMM, batched: for batch index z (z_lo = z % Z0,

@@ -1,0 +1,74 @@
+"""The streamed x/y and z passes (stream.hip) against the separate passes
+(DAGE_APPLY_STREAM=0) and the oracle, at sizes around the 16-point tiles,
+rectangular grids, and axes where the banded ring and the full kernel meet.
+
+Both paths sum the same products (the flushed matrices' zeros are skipped by
+either), in another order: at every point they differ by at most
+2 (nx + ny + nz + T + 3) 2^-53 times the sum of the products' magnitudes.
+"""
+import numpy as np
+import pytest
+
+import dage_amd
+import oracle as O
+from _helpers import rel_maxdiff
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # cells per input axis, per output axis (None: same grid), nlip, cell length
+    ((1, 2, 4), None, 2, 0.4),
+    ((14, 15, 16), None, 2, 0.4),                 # 15, 16, 17 points
+    ((30, 31, 32), None, 2, 0.3),
+    ((47, 16, 33), None, 2, 0.3),
+    ((8, 10, 12), (3, 5, 2), 5, 0.5),             # rectangular: always the full kernel
+    ((24, 4, 10), (4, 24, 11), 4, 0.5),
+    ((16, 16, 16), None, 5, 0.6),                 # 65: rings of 3 beside the full 5
+    ((52, 22, 4), None, 5, 0.6),                  # 209 points: the widest full kernel is too small
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_streamed_passes(ctx, monkeypatch, case):
+    cin, cout, nlip, h = CASES[case]
+    lo = [-0.5 * h * n + 0.05 * k for k, n in enumerate(cin)]
+    ain = [O.Axis(a, np.full(n, h), nlip) for a, n in zip(lo, cin)]
+    aout = ain if cout is None else [O.Axis(a + 0.3 * h, np.full(n, 0.8 * h), nlip)
+                                     for a, n in zip(lo, cout)]
+    rng = np.random.default_rng(60 + case)
+    x = np.asfortranarray(rng.standard_normal([a.n for a in ain]))
+    q = dage_amd.GaussQuad(nlin=12, nlog=12, tlin=2.0, tlog=300.0)
+    w = O.coulomb_weights(q.tw)
+    F = [O.exponentials(i, o, q.tp, False) for i, o in zip(ain, aout)]  # (out, in, t)
+    S = np.zeros([a.n for a in aout])
+    for t in range(len(q.tp)):
+        v = np.abs(x)
+        for axis in range(3):
+            v = np.moveaxis(np.tensordot(np.abs(F[axis][:, :, t]), v, axes=(1, axis)), 0, axis)
+        S += abs(w[t]) * v
+
+    def grid(axes):
+        return dage_amd.Grid3D(ctx, [a.qmin for a in axes], [a.steps for a in axes], nlip)
+
+    gin = grid(ain)
+    gout = gin if cout is None else grid(aout)
+    op = dage_amd.Coulomb3D(ctx, gin, gout, q, coda=False)
+    a = dage_amd.DeviceCube(ctx, x.shape, x)
+    b = dage_amd.DeviceCube(ctx, S.shape)
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("DAGE_APPLY_STREAM", mode)
+        ctx.profile(True)
+        op.transform_cuda_cube(a, b)
+        streamed = ctx.profile_query("gemm_f64_xymode")[1]
+        ctx.profile(False)
+        assert (streamed > 0) == (mode == "1")
+        got[mode] = b.download().copy()
+    n = sum(i.n for i in ain) + len(q.tp) + 3
+    diff = np.abs(got["1"] - got["0"])
+    print(f"case {case}: {x.shape} -> {S.shape}, {(diff / (2 * n * 2.0 ** -53 * S)).max():.3f} of the "
+          f"bound, {diff.max() / np.abs(got['0']).max():.2e} of max|out|")
+    assert np.all(diff <= 2 * n * 2.0 ** -53 * S)
+    ref = O.transform_cube(F[0], F[1].transpose(1, 0, 2).copy("F"), F[2].transpose(1, 0, 2).copy("F"),
+                           w, 0.0, x, add_coda=False)
+    assert rel_maxdiff(got["1"], ref) < 1e-10

@@ -20,10 +20,8 @@
 // Algorithmic work: 2*16*16*27 = 13824 FLOPs per voxel (dense, as FP32);
 // HBM roofline 128 bytes per voxel (16 channels in and out, FP32).
 //
-// Layers with 1 or 2 channels on a side run as FP32 VALU kernels; the
-// backward filter stages, per output x-row and per dz, the 3 neighbouring
-// input rows of every channel in LDS, and every thread owns one (cout, cin)
-// pair's 27 taps.
+// Forward and backward-data layers with 1 or 2 channels on a side run as FP32
+// VALU kernels, the filter gradients on FP32 MFMA.
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>
@@ -350,78 +348,367 @@ int launch_conv16(dage_ctx ctx, int nx, int ny, int nz, const float *in, const u
     return DAGE_OK;
 }
 
-// Filter gradient, stage 1: block b takes x-rows (y, z) in [b*rows, ...);
-// thread t = o*cin + c accumulates gW[o][c][0..26] and (c == 0) gb[o].  Per
-// row and per dz the 3 input rows (y-1..y+1) of every channel are staged in
-// LDS with a one-point halo in x.
-__global__ void __launch_bounds__(256) conv_bwd_filter_kernel(const float *in, const float *gout,
-                                                              int cin, int cout, int nx, int ny,
-                                                              int nz, int rows_per_block,
-                                                              float *part) {
-    extern __shared__ float sm[];
-    const int W = nx + 2;
-    float *sin_ = sm;                  // [cin][3][W]
-    float *sgo = sm + cin * 3 * W;     // [cout][nx]
-    const int tid = threadIdx.x;
-    const int o = tid / cin, c = tid % cin;
-    const bool active = tid < cin * cout;
-    float acc[27];
-#pragma unroll
-    for (int t = 0; t < 27; ++t) acc[t] = 0.0f;
-    float accb = 0.0f;
+// Filter gradient gW[o][c][t] = sum_p gout[o][p] in[c][p + off(t)] as matrix
+// products over the voxels on FP32 MFMA (v_mfma_f32_16x16x4f32: lane l holds
+// A(l%16, l/16) and B(l/16, l%16); result register r of lane l is
+// D(4(l/16)+r, l%16)): exact FP32 products, FP32 sums.  A block takes a range
+// of x-rows (y, z) of one x chunk and walks along y with the rows it needs in
+// LDS: one barrier per row, the next rows on their way in registers.  A
+// channel row in LDS has kRowS floats (4 times an odd number: 16 channels at
+// this stride and 4 segments an odd number apart fall on different banks).
+// Sums run per wavefront over its block's rows, then over the wavefronts and
+// (sum_blocks_kernel) the blocks, in a fixed order.
+//
+// Both replace a VALU kernel whose threads owned one (o, c) pair's 27 taps:
+// bound by its LDS reads (two per multiply-add of a tap) and, with few
+// channels, by idle threads.  129^3, 16 -> 16: 900 -> 314 us (29.7 GFLOP,
+// 195 us at the 152 TFLOP/s of a large FP32 product; the matrix cores are busy
+// 67 % of the time, the rest is the row barriers and the segments' padding
+// from 129 to 144 points); 2 -> 16: 900 -> 86, 16 -> 1: 900 -> 45 us (31 us for
+// the bytes at 4.7 TB/s).
+constexpr int kSegL = 9;               // longest x segment of a lane group
+constexpr int kRowS = 16 * kSegL + 4;  // 148
+constexpr int kStage = 3;              // 64-float loads that cover a row
+
+// A channel row of a volume as a buffer: loads outside [0, nx), or of a row
+// or channel that does not exist, return zero.
+__device__ inline __amdgpu_buffer_rsrc_t row_buffer(const float *p, long vol, int c, int nc, int y,
+                                                    int z, int nx, int ny, int nz) {
+    const bool ok = c < nc && y >= 0 && y < ny && z >= 0 && z < nz;
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p + (ok ? (long)c * vol + (long)nx * (y + (long)ny * z) : 0)), 0,
+        ok ? 4 * nx : 0, 0x00027000);
+}
+__device__ inline float row_load(__amdgpu_buffer_rsrc_t r, int x) {
+    const unsigned off = x < 0 ? 0x80000000u : 4u * (unsigned)x;
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
+}
+
+// Up to 16 x 16 channels.  Wavefront (dz, w) of 12 sums the 9 taps of one dz
+// over segment 4w + l/16 (L points) of each row: A = gout (16 o x 4 voxels),
+// B = in (4 voxels x 16 c) of the tap's row; along the segment one LDS read
+// per row feeds the three dx taps in turn.
+template <int L>
+__global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, const float *gout,
+                                                               int cin, int cout, int nx, int ny,
+                                                               int nz, int rows_per_block,
+                                                               float *part) {
+    constexpr int ROW = 16 * kRowS;
+    // input rows (dz, y & 3), then output rows y & 1; at the end the sums
+    __shared__ float sm[14 * ROW];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int dz = wave >> 2, w = wave & 3;
+    const int n = lane & 15, k = lane >> 4;
+    const int x0 = blockIdx.y * 16 * L;
     const long vol = (long)nx * ny * nz;
     const long nrows = (long)ny * nz;
     const long r0 = (long)blockIdx.x * rows_per_block;
-    const long r1 = r0 + rows_per_block < nrows ? r0 + rows_per_block : nrows;
-    for (long row = r0; row < r1; ++row) {
-        const int y = (int)(row % ny), z = (int)(row / ny);
+    const long r1 = min(nrows, r0 + rows_per_block);
+    const int start = (4 * w + k) * L;
+
+    // A row's sums start at zero and are added to the block's after it: chains
+    // of L matrix products and of the rows instead of their product (one
+    // accumulator for all rows had 3 times the error).
+    f4 sum[9];
 #pragma unroll
-        for (int kz = 0; kz < 3; ++kz) {
-            __syncthreads();
-            const int zz = z + kz - 1;
-            for (int e = tid; e < cin * 3 * W; e += 256) {
-                const int cc = e / (3 * W);
-                const int rem = e - cc * 3 * W;
-                const int ky = rem / W, xx = rem % W - 1;
-                const int yy = y + ky - 1;
-                const bool ok = xx >= 0 && xx < nx && yy >= 0 && yy < ny && zz >= 0 && zz < nz;
-                sin_[e] = ok ? in[(long)cc * vol + xx + (long)nx * (yy + (long)ny * zz)] : 0.0f;
-            }
-            if (kz == 0)
-                for (int e = tid; e < cout * nx; e += 256) {
-                    const int oo = e / nx, xx = e % nx;
-                    sgo[e] = gout[(long)oo * vol + xx + (long)nx * (y + (long)ny * z)];
-                }
-            __syncthreads();
-            if (active) {
-                const float *go = sgo + o * nx;
-                const float *ic = sin_ + c * 3 * W;
-                for (int x = 0; x < nx; ++x) {
-                    const float g = go[x];
-                    if (kz == 0 && c == 0) accb += g;
+    for (int t = 0; t < 9; ++t) sum[t] = f4{0.f, 0.f, 0.f, 0.f};
+    float sumb = 0.0f;
+
+    // staging: wavefront `wave` takes channel rows wave, wave + 12, ... of the
+    // 48 input rows and of the 16 output rows
+    float ri[4][kStage], ro[2][kStage];
+    auto load_in = [&](int y, int z) {
 #pragma unroll
-                    for (int ky = 0; ky < 3; ++ky)
+        for (int q = 0; q < 4; ++q) {
+            const int e = wave + 12 * q;
+            const __amdgpu_buffer_rsrc_t r = row_buffer(in, vol, e & 15, cin, y, z + (e >> 4) - 1, nx, ny, nz);
 #pragma unroll
-                        for (int dx = 0; dx < 3; ++dx)
-                            acc[9 * kz + 3 * ky + dx] += g * ic[ky * W + x + dx];
-                }
+            for (int h = 0; h < kStage; ++h) ri[q][h] = row_load(r, x0 - 1 + lane + 64 * h);
+        }
+    };
+    auto store_in = [&](int y) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e = wave + 12 * q;
+            float *d = sm + (4 * (e >> 4) + (y & 3)) * ROW + (e & 15) * kRowS;
+#pragma unroll
+            for (int h = 0; h < kStage; ++h)
+                if (lane + 64 * h < kRowS) d[lane + 64 * h] = ri[q][h];
+        }
+    };
+    auto load_out = [&](int y, int z) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int e = wave + 12 * q;
+            const __amdgpu_buffer_rsrc_t r = row_buffer(gout, vol, e, cout, y, z, nx, ny, nz);
+#pragma unroll
+            for (int h = 0; h < kStage; ++h) {
+                const int x = lane + 64 * h;
+                ro[q][h] = row_load(r, x < 16 * L ? x0 + x : -1);
             }
         }
-    }
-    if (active) {
-        float *pp = part + (long)blockIdx.x * (cout * cin * 27 + cout);
+    };
+    auto store_out = [&](int y) {
 #pragma unroll
-        for (int t = 0; t < 27; ++t) pp[(o * cin + c) * 27 + t] = acc[t];
-        if (c == 0) pp[cout * cin * 27 + o] = accb;
+        for (int q = 0; q < 2; ++q) {
+            const int e = wave + 12 * q;
+            float *d = sm + (12 + (y & 1)) * ROW + e * kRowS;
+#pragma unroll
+            for (int h = 0; h < kStage; ++h)
+                if (e < 16 && lane + 64 * h < kRowS) d[lane + 64 * h] = ro[q][h];
+        }
+    };
+
+    for (long row = r0; row < r1;) {
+        const int z = (int)(row / ny), ya = (int)(row - (long)z * ny);
+        const int yb = (int)min((long)ny, ya + r1 - row);  // rows [ya, yb) of plane z
+        for (int y = ya - 1; y <= ya + 1; ++y) {
+            load_in(y, z);
+            store_in(y);
+        }
+        load_out(ya, z);
+        store_out(ya);
+        __syncthreads();
+        for (int y = ya; y < yb; ++y) {
+            // row y + 2 replaces y - 2, output row y + 1 replaces y - 1
+            load_in(y + 2, z);
+            load_out(y + 1, z);
+            const float *go = sm + (12 + (y & 1)) * ROW + n * kRowS + start;
+            const float *ir[3];
+            float v0[3], v1[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                ir[d] = sm + (4 * dz + ((y + d - 1) & 3)) * ROW + n * kRowS + start;
+                v0[d] = ir[d][0];
+                v1[d] = ir[d][1];
+            }
+            f4 acc[9];
+#pragma unroll
+            for (int t = 0; t < 9; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+            float accb = 0.0f;
+#pragma unroll
+            for (int x = 0; x < L; ++x) {
+                const float g = go[x];
+                accb += g;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const float v2 = ir[d][x + 2];
+                    acc[3 * d] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v0[d], acc[3 * d], 0, 0, 0);
+                    acc[3 * d + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v1[d], acc[3 * d + 1], 0, 0, 0);
+                    acc[3 * d + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v2, acc[3 * d + 2], 0, 0, 0);
+                    v0[d] = v1[d];
+                    v1[d] = v2;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 9; ++t) sum[t] += acc[t];
+            sumb += accb;
+            store_in(y + 2);
+            store_out(y + 1);
+            __syncthreads();
+        }
+        row += yb - ya;
+    }
+    // sum over the four segments' wavefronts
+    float *red = sm + (w * 3 + dz) * 36 * 64 + lane, *redb = sm + 12 * 36 * 64;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[(t * 4 + r) * 64] = sum[t][r];
+    if (dz == 1) redb[w * 64 + lane] = sumb;
+    __syncthreads();
+    const int len = cout * cin * 27 + cout;
+    float *pp = part + ((long)blockIdx.y * gridDim.x + blockIdx.x) * len;
+    for (int e = tid; e < 3 * 36 * 64; e += 768) {
+        const int l = e & 63, q = e >> 6, t = q >> 2;
+        const int o = 4 * (l >> 4) + (q & 3), c = l & 15;
+        float s = 0.0f;
+        for (int v = 0; v < 4; ++v) s += sm[v * 3 * 36 * 64 + e];
+        if (o < cout && c < cin) pp[(o * cin + c) * 27 + t] = s;
+    }
+    if (tid < cout) {
+        float s = 0.0f;
+        for (int v = 0; v < 16; ++v) s += redb[16 * v + tid];
+        pp[cout * cin * 27 + tid] = s;
     }
 }
 
-__global__ void __launch_bounds__(256) sum_blocks_kernel(const float *part, int nblocks, int len,
-                                                         float *out) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < len; i += gridDim.x * blockDim.x) {
+// One side with CH = 1 or 2 channels (Y), the other (X) with up to 16:
+// R[m][col] = sum_p X[m][p] Y[ch][p + off(t)], col = 27 ch + t, and
+// col = 27 CH the plain sum of X.  The taps are the columns of B, so a
+// 4-voxel step costs 2 CH MFMAs.  X = gout (swap = 0): R is gW and the last
+// column gb.  X = in (swap = 1): gW[ch][m][26 - t] = R[m][27 ch + t], and
+// gb[ch] is summed from the staged rows of Y.
+template <int CH>
+__global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, const float *Y,
+                                                              int nm, int nx, int ny, int nz,
+                                                              int width, int swap,
+                                                              int rows_per_block, float *part) {
+    constexpr int NT = 2 * CH, YQ = (3 * CH + 3) / 4;
+    constexpr int RED = NT * 4 * 64;
+    // X rows (y & 1, m), at the end the sums; Y rows (dz, y & 3, ch), a row
+    // of ones and one of zeros (the columns past the taps)
+    __shared__ float sx[2 * 16 * kRowS];
+    __shared__ float sy[(12 * CH + 2) * kRowS];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, k = lane >> 4;
+    const int x0 = blockIdx.y * width;
+    const long vol = (long)nx * ny * nz;
+    const long nrows = (long)ny * nz;
+    const long r0 = (long)blockIdx.x * rows_per_block;
+    const long r1 = min(nrows, r0 + rows_per_block);
+
+    f4 sum[NT];
+    float accb[CH];
+    int ty[NT], to[NT];  // this lane's column: input row y + ty - 1 (ty < 0: any), offset
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        sum[j] = f4{0.f, 0.f, 0.f, 0.f};
+        const int col = 16 * j + n, ch = min(col / 27, CH - 1), t = (col - 27 * ch) % 27;
+        const bool tap = col < 27 * CH;
+        ty[j] = tap ? t / 3 % 3 : -1;
+        to[j] = (tap ? 4 * (t / 9) * CH + ch : 12 * CH + (col > 27 * CH)) * kRowS + (tap ? t % 3 : 0) + k;
+    }
+    if (tid < kRowS) {
+        sy[12 * CH * kRowS + tid] = 1.0f;
+        sy[(12 * CH + 1) * kRowS + tid] = 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) accb[c] = 0.0f;
+
+    float rx[4][kStage], ry[YQ][kStage];
+    auto load_x = [&](int y, int z) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const __amdgpu_buffer_rsrc_t r = row_buffer(X, vol, wave + 4 * q, nm, y, z, nx, ny, nz);
+#pragma unroll
+            for (int h = 0; h < kStage; ++h) {
+                const int x = lane + 64 * h;
+                rx[q][h] = row_load(r, x < width ? x0 + x : -1);
+            }
+        }
+    };
+    auto store_x = [&](int y) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int h = 0; h < kStage; ++h)
+                if (lane + 64 * h < kRowS) sx[(16 * (y & 1) + wave + 4 * q) * kRowS + lane + 64 * h] = rx[q][h];
+    };
+    auto load_y = [&](int y, int z) {
+#pragma unroll
+        for (int q = 0; q < YQ; ++q) {
+            const int e = wave + 4 * q;
+            const __amdgpu_buffer_rsrc_t r =
+                row_buffer(Y, vol, e % CH, e < 3 * CH ? CH : 0, y, z + e / CH - 1, nx, ny, nz);
+#pragma unroll
+            for (int h = 0; h < kStage; ++h) ry[q][h] = row_load(r, x0 - 1 + lane + 64 * h);
+        }
+    };
+    auto store_y = [&](int y) {
+#pragma unroll
+        for (int q = 0; q < YQ; ++q) {
+            const int e = wave + 4 * q;
+            if (e >= 3 * CH) continue;
+            float *d = sy + ((4 * (e / CH) + (y & 3)) * CH + e % CH) * kRowS;
+#pragma unroll
+            for (int h = 0; h < kStage; ++h)
+                if (lane + 64 * h < kRowS) d[lane + 64 * h] = ry[q][h];
+        }
+    };
+
+    for (long row = r0; row < r1;) {
+        const int z = (int)(row / ny), ya = (int)(row - (long)z * ny);
+        const int yb = (int)min((long)ny, ya + r1 - row);
+        for (int y = ya - 1; y <= ya + 1; ++y) {
+            load_y(y, z);
+            store_y(y);
+        }
+        load_x(ya, z);
+        store_x(ya);
+        __syncthreads();
+        for (int y = ya; y < yb; ++y) {
+            load_y(y + 2, z);
+            load_x(y + 1, z);
+            if (swap && tid < width) {
+#pragma unroll
+                for (int c = 0; c < CH; ++c)
+                    // (past the last column the row holds zeros)
+                    accb[c] += x0 + tid < nx ? sy[((4 + (y & 3)) * CH + c) * kRowS + tid + 1] : 0.0f;
+            }
+            const float *xr = sx + (16 * (y & 1) + n) * kRowS + k;
+            const float *yr[NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                yr[j] = sy + (ty[j] < 0 ? 0 : ((y + ty[j] - 1) & 3) * CH * kRowS) + to[j];
+            f4 acc[NT];  // this row's sums (see conv_filter_mfma_kernel)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 3
+            for (int x = 4 * wave; x < width; x += 16) {
+                const float a = xr[x];
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, yr[j][x], acc[j], 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) sum[j] += acc[j];
+            store_y(y + 2);
+            store_x(y + 1);
+            __syncthreads();
+        }
+        row += yb - ya;
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sx[wave * RED + (j * 4 + r) * 64 + lane] = sum[j][r];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) sy[c * 256 + tid] = accb[c];
+    __syncthreads();
+    const int cout = swap ? CH : nm, cin = swap ? nm : CH;
+    float *pp = part + ((long)blockIdx.y * gridDim.x + blockIdx.x) * (cout * cin * 27 + cout);
+    for (int e = tid; e < NT * 4 * 64; e += 256) {
+        const int l = e & 63, q = e >> 6;
+        const int m = 4 * (l >> 4) + (q & 3), col = 16 * (q >> 2) + (l & 15);
+        const float s = ((sx[e] + sx[RED + e]) + sx[2 * RED + e]) + sx[3 * RED + e];
+        if (m >= nm || col > 27 * CH) continue;
+        const int ch = col / 27, t = col - 27 * ch;
+        if (col == 27 * CH) {
+            if (!swap) pp[cout * cin * 27 + m] = s;
+        } else {
+            pp[swap ? (ch * nm + m) * 27 + 26 - t : (m * CH + ch) * 27 + t] = s;
+        }
+    }
+    if (swap && wave < CH) {  // a fixed tree over the columns
         float s = 0.0f;
-        for (int b = 0; b < nblocks; ++b) s += part[(long)b * len + i];
-        out[i] = s;
+        for (int h = 0; h < 4; ++h) s += sy[256 * wave + lane + 64 * h];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (lane == 0) pp[cout * cin * 27 + wave] = s;
+    }
+}
+
+// Sum of the blocks' partials, 32 entries per block: 8 thread rows take every
+// eighth block, then a fixed sum over the rows, in FP64 (the serial FP32 loop
+// over 1024 blocks took 230 us at 6928 entries, this one 9).  The first
+// nw sums go to gw, the others to gb.
+__global__ void __launch_bounds__(256) sum_blocks_kernel(const float *part, int nblocks, int len,
+                                                         int nw, float *gw, float *gb) {
+    __shared__ double red[8][32];
+    const int col = threadIdx.x & 31, g = threadIdx.x >> 5;
+    const int i = blockIdx.x * 32 + col;
+    double s = 0.0;
+    if (i < len)
+#pragma unroll 4
+        for (int b = g; b < nblocks; b += 8) s += part[(long)b * len + i];
+    red[g][col] = s;
+    __syncthreads();
+    if (g == 0 && i < len) {
+#pragma unroll
+        for (int q = 1; q < 8; ++q) s += red[q][col];
+        (i < nw ? gw : gb - nw)[i] = (float)s;
     }
 }
 
@@ -556,25 +843,52 @@ int dage_conv3d_backward_filter(dage_ctx ctx, int nx, int ny, int nz, int cin, i
     const size_t smem = sizeof(float) * ((size_t)cin * 3 * (nx + 2) + (size_t)cout * nx);
     DAGE_REQUIRE(smem <= 64 * 1024, DAGE_ERR_UNSUPPORTED, "x extent %d too long for one block",
                  nx);
+    // x chunks of at most 16*kSegL columns; blocks of rows for one block per
+    // CU (16 x 16 channels: 132 KB of LDS) or four (the few-channel kernel,
+    // bound by its loads)
+    const bool few = std::min(cin, cout) <= 2;
+    const int chunks = (nx + 16 * kSegL - 1) / (16 * kSegL);
+    const int width = (nx + chunks - 1) / chunks;
+    int L = (width + 15) / 16;
+    if (L % 4 == 0) ++L;  // segments a multiple of 4 apart share banks
     const long nrows = (long)ny * nz;
-    const int rows = (int)std::max<long>(1, (nrows + 1023) / 1024);
-    const int nblocks = (int)((nrows + rows - 1) / rows);
-    const int len = cout * cin * 27 + cout;
-    const size_t bpart = sizeof(float) * (size_t)nblocks * len;
+    const int want = std::max(1, (few ? 1024 : 256) / chunks);
+    const int rows = (int)((nrows + want - 1) / want);
+    const int rblocks = (int)((nrows + rows - 1) / rows), nblocks = rblocks * chunks;
+    const int nw = cout * cin * 27, len = nw + cout;
     void *scr = nullptr;
-    DAGE_TRY(ctx_scratch(ctx, (bpart + 255) / 256 * 256 + sizeof(float) * len, &scr));
+    DAGE_TRY(ctx_scratch(ctx, sizeof(float) * (size_t)nblocks * len, &scr));
     float *part = static_cast<float *>(scr);
-    float *sums = reinterpret_cast<float *>(static_cast<char *>(scr) + (bpart + 255) / 256 * 256);
-    hipLaunchKernelGGL(conv_bwd_filter_kernel, dim3(nblocks), dim3(256), smem, ctx->stream, in,
-                       gout, cin, cout, nx, ny, nz, rows, part);
+    const dim3 grid(rblocks, chunks);
+    if (!few) {
+        auto run = [&](auto l) {
+            hipLaunchKernelGGL(conv_filter_mfma_kernel<decltype(l)::value>, grid, dim3(768), 0,
+                               ctx->stream, in, gout, cin, cout, nx, ny, nz, rows, part);
+        };
+        switch (L) {
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        case 5: run(std::integral_constant<int, 5>{}); break;
+        case 6: run(std::integral_constant<int, 6>{}); break;
+        case 7: run(std::integral_constant<int, 7>{}); break;
+        default: run(std::integral_constant<int, kSegL>{}); break;
+        }
+    } else {
+        const int swap = cin > 2, ch = swap ? cout : cin;
+        const float *X = swap ? in : gout, *Y = swap ? gout : in;
+        const int nm = swap ? cin : cout;
+        if (ch == 1)
+            hipLaunchKernelGGL(conv_filter_few_kernel<1>, grid, dim3(256), 0, ctx->stream, X, Y, nm,
+                               nx, ny, nz, width, swap, rows, part);
+        else
+            hipLaunchKernelGGL(conv_filter_few_kernel<2>, grid, dim3(256), 0, ctx->stream, X, Y, nm,
+                               nx, ny, nz, width, swap, rows, part);
+    }
     DAGE_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(sum_blocks_kernel, dim3((len + 255) / 256), dim3(256), 0, ctx->stream,
-                       part, nblocks, len, sums);
+    hipLaunchKernelGGL(sum_blocks_kernel, dim3((len + 31) / 32), dim3(256), 0, ctx->stream, part,
+                       nblocks, len, nw, gw, gb);
     DAGE_HIP_CHECK(hipGetLastError());
-    DAGE_HIP_CHECK(hipMemcpyAsync(gw, sums, sizeof(float) * (len - cout), hipMemcpyDeviceToDevice,
-                                  ctx->stream));
-    DAGE_HIP_CHECK(hipMemcpyAsync(gb, sums + (len - cout), sizeof(float) * cout,
-                                  hipMemcpyDeviceToDevice, ctx->stream));
     return DAGE_OK;
 }
 

@@ -204,7 +204,7 @@ int dage_operator_apply_device_strided(dage_operator op, const double *in, int l
  * its intermediates in a fixed per-GPU scratch array of
  * dage_operator_noalloc_limit() bytes (128 MiB) that the library holds for
  * the life of the process.  The t-chunk shrinks to fit; when the
- * intermediates of one t-point (8*nxo*nyo*nzi bytes with the fused x/y pass,
+ * intermediates of one t-point (8*nxo*(nyi + nyo)*nzi bytes,
  * plus the z-pass partials) do not fit, DAGE_ERR_ARG is returned and nothing
  * is launched.  Calls no allocator.  Every call on one GPU shares that GPU's
  * array, so calls that overlap on one GPU (other streams, other contexts,

@@ -946,7 +946,6 @@ int dage_bubbles_destroy(dage_bubbles b) {
         if (h.d_tab) (void)hipFree(h.d_tab);
     }
     if (b->d_desc) (void)hipFree(b->d_desc);
-    if (b->d_pack) (void)hipFree(b->d_pack);
     delete b;
     ctx_release(ctx);
     return DAGE_OK;

@@ -139,7 +139,6 @@ struct BubbleDev {
     const double *celld;   // ncell cell starts
     const double *steps;   // ncell cell steps
     const double *f;       // npts x (lmax+1)^2, r^k folded in, point fastest
-    double *pack;          // the same by cell, for the inject kernels (inject.hip)
     int ncell, npts;
     // cell-lookup table: ctab[k] = cell (1-based) holding r = k*qmax/kCellTab
     const int *ctab;
@@ -169,8 +168,6 @@ struct dage_bubbles_s {
     int nbub = 0, lmax = 0, k = 0, nlip = 7;
     std::vector<dage::BubbleHost> host;
     dage::BubbleDev *d_desc = nullptr;
-    double *d_pack = nullptr;  // every bubble's BubbleDev::pack
-    size_t pack_size = 0;
     bool dirty = true;
     int nlm() const { return (lmax + 1) * (lmax + 1); }
     // raw radial values f (npts x nlm, point fastest) of bubble i

@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
     const long nrows = (long)ny * nz;
     const long r0 = (long)blockIdx.x * rows_per_block;
     const long r1 = min(nrows, r0 + rows_per_block);
-    const int start = (4 * w + k) * L;
+    const int start = (4 * w + k) * L, last = nx - x0 - start;
 
     // A row's sums start at zero and are added to the block's after it: chains
     // of L matrix products and of the rows instead of their product (one
@@ -480,7 +480,9 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 ir[d] = sm + (4 * dz + ((y + d - 1) & 3)) * ROW + n * kRowS + start;
-                v0[d] = ir[d][0];
+                // the left tap of the first padding column is in[nx - 1]; as
+                // zero it cannot turn an infinity there into a NaN
+                v0[d] = 0 < last ? ir[d][0] : 0.0f;
                 v1[d] = ir[d][1];
             }
             f4 acc[9];
@@ -497,7 +499,7 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
                     acc[3 * d] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v0[d], acc[3 * d], 0, 0, 0);
                     acc[3 * d + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v1[d], acc[3 * d + 1], 0, 0, 0);
                     acc[3 * d + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v2, acc[3 * d + 2], 0, 0, 0);
-                    v0[d] = v1[d];
+                    v0[d] = x + 1 < last ? v1[d] : 0.0f;
                     v1[d] = v2;
                 }
             }

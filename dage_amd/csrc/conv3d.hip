@@ -539,14 +539,14 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
 // One side with CH = 1 or 2 channels (Y), the other (X) with up to 16:
 // R[m][col] = sum_p X[m][p] Y[ch][p + off(t)], col = 27 ch + t, and
 // col = 27 CH the plain sum of X.  The taps are the columns of B, so a
-// 4-voxel step costs 2 CH MFMAs.  X = gout (swap = 0): R is gW and the last
-// column gb.  X = in (swap = 1): gW[ch][m][26 - t] = R[m][27 ch + t], and
+// 4-voxel step costs 2 CH MFMAs.  X = gout: R is gW and the last
+// column gb.  X = in (SWAP): gW[ch][m][26 - t] = R[m][27 ch + t], and
 // gb[ch] is summed from the staged rows of Y.
-template <int CH>
+template <int CH, bool SWAP>
 __global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, const float *Y,
                                                               int nm, int nx, int ny, int nz,
-                                                              int width, int swap,
-                                                              int rows_per_block, float *part) {
+                                                              int width, int rows_per_block,
+                                                              float *part) {
     constexpr int NT = 2 * CH, YQ = (3 * CH + 3) / 4;
     constexpr int RED = NT * 4 * 64;
     // X rows (y & 1, m), at the end the sums; Y rows (dz, y & 3, ch), a row
@@ -562,15 +562,25 @@ __global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, co
     const long r0 = (long)blockIdx.x * rows_per_block;
     const long r1 = min(nrows, r0 + rows_per_block);
 
+    // An infinity of Y or X meets no zero of the padding past the row, of the
+    // next chunk or, where X = in, outside the volume: the columns of
+    // [xlo, xhi) have all their neighbours in the row and run in whole steps
+    // of 4, the others in a masked step; X = in: the first and the last column
+    // without the taps outside, and a row's sums without the rows outside.
+    const int xend = min(width, nx - x0), xlo = SWAP && x0 == 0;
+    const int xhi = xend - (SWAP && x0 + xend == nx);
     f4 sum[NT];
     float accb[CH];
-    int ty[NT], to[NT];  // this lane's column: input row y + ty - 1 (ty < 0: any), offset
+    // this lane's column: input row y + ty - 1 (ty < 0: any), offset, and its
+    // place among the 9 rows (9: none) with 16 times its place in the row
+    int ty[NT], to[NT], tc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         sum[j] = f4{0.f, 0.f, 0.f, 0.f};
         const int col = 16 * j + n, ch = min(col / 27, CH - 1), t = (col - 27 * ch) % 27;
         const bool tap = col < 27 * CH;
         ty[j] = tap ? t / 3 % 3 : -1;
+        tc[j] = tap ? t / 3 + 16 * (t % 3) : 9 + 16;
         to[j] = (tap ? 4 * (t / 9) * CH + ch : 12 * CH + (col > 27 * CH)) * kRowS + (tap ? t % 3 : 0) + k;
     }
     if (tid < kRowS) {
@@ -634,7 +644,7 @@ __global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, co
         for (int y = ya; y < yb; ++y) {
             load_y(y + 2, z);
             load_x(y + 1, z);
-            if (swap && tid < width) {
+            if (SWAP && tid < width) {
 #pragma unroll
                 for (int c = 0; c < CH; ++c)
                     // (past the last column the row holds zeros)
@@ -646,17 +656,38 @@ __global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, co
             for (int j = 0; j < NT; ++j)
                 yr[j] = sy + (ty[j] < 0 ? 0 : ((y + ty[j] - 1) & 3) * CH * kRowS) + to[j];
             f4 acc[NT];  // this row's sums (see conv_filter_mfma_kernel)
+            // a step apart: wavefront 0 the columns 1..3, 1 those from xs on,
+            // 2 the first and 3 the last column
+            const int xs = xhi & ~3;
+            {
+                const int x = wave == 1 ? xs : (wave == 3 ? xend - 1 : 0), c = x + k;
+                const bool on = wave == 0   ? xlo && xs > 0 && k > 0
+                                : wave == 1 ? c >= xlo && c < xhi
+                                : wave == 2 ? xlo && k == 0
+                                            : xhi < xend && nx > 1 && k == 0;
+                const bool first = SWAP && wave == 2, last = SWAP && (wave == 3 || (first && nx == 1));
+                const float a = on ? xr[x] : 0.0f;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < NT; ++j) {
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        a, on ? yr[j][x] : 0.0f, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    const int dx = tc[j] >> 4;
+                    if ((first && dx == 0) || (last && dx == 2)) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
 #pragma unroll 3
-            for (int x = 4 * wave; x < width; x += 16) {
+            for (int x = 4 * wave + (wave < xlo ? 16 : 0); x < xs; x += 16) {
                 const float a = xr[x];
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
                     acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, yr[j][x], acc[j], 0, 0, 0);
             }
+            // bit 3 dz + dy: the row of that tap exists
+            const int yok = (y > 0) + 2 + 4 * (y + 1 < ny);
+            const int rows = (z > 0 ? yok : 0) + 8 * yok + (z + 1 < nz ? 64 * yok : 0) + 512;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) sum[j] += acc[j];
+            for (int j = 0; j < NT; ++j)
+                if (!SWAP || ((rows >> (tc[j] & 15)) & 1)) sum[j] += acc[j];
             store_y(y + 2);
             store_x(y + 1);
             __syncthreads();
@@ -670,7 +701,7 @@ __global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, co
 #pragma unroll
     for (int c = 0; c < CH; ++c) sy[c * 256 + tid] = accb[c];
     __syncthreads();
-    const int cout = swap ? CH : nm, cin = swap ? nm : CH;
+    const int cout = SWAP ? CH : nm, cin = SWAP ? nm : CH;
     float *pp = part + ((long)blockIdx.y * gridDim.x + blockIdx.x) * (cout * cin * 27 + cout);
     for (int e = tid; e < NT * 4 * 64; e += 256) {
         const int l = e & 63, q = e >> 6;
@@ -679,12 +710,12 @@ __global__ void __launch_bounds__(256) conv_filter_few_kernel(const float *X, co
         if (m >= nm || col > 27 * CH) continue;
         const int ch = col / 27, t = col - 27 * ch;
         if (col == 27 * CH) {
-            if (!swap) pp[cout * cin * 27 + m] = s;
+            if (!SWAP) pp[cout * cin * 27 + m] = s;
         } else {
-            pp[swap ? (ch * nm + m) * 27 + 26 - t : (m * CH + ch) * 27 + t] = s;
+            pp[SWAP ? (ch * nm + m) * 27 + 26 - t : (m * CH + ch) * 27 + t] = s;
         }
     }
-    if (swap && wave < CH) {  // a fixed tree over the columns
+    if (SWAP && wave < CH) {  // a fixed tree over the columns
         float s = 0.0f;
         for (int h = 0; h < 4; ++h) s += sy[256 * wave + lane + 64 * h];
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
@@ -877,15 +908,18 @@ int dage_conv3d_backward_filter(dage_ctx ctx, int nx, int ny, int nz, int cin, i
         default: run(std::integral_constant<int, kSegL>{}); break;
         }
     } else {
-        const int swap = cin > 2, ch = swap ? cout : cin;
+        const bool swap = cin > 2;
         const float *X = swap ? in : gout, *Y = swap ? gout : in;
         const int nm = swap ? cin : cout;
-        if (ch == 1)
-            hipLaunchKernelGGL(conv_filter_few_kernel<1>, grid, dim3(256), 0, ctx->stream, X, Y, nm,
-                               nx, ny, nz, width, swap, rows, part);
-        else
-            hipLaunchKernelGGL(conv_filter_few_kernel<2>, grid, dim3(256), 0, ctx->stream, X, Y, nm,
-                               nx, ny, nz, width, swap, rows, part);
+        auto run = [&](auto ch, auto sw) {
+            hipLaunchKernelGGL((conv_filter_few_kernel<decltype(ch)::value, decltype(sw)::value>),
+                               grid, dim3(256), 0, ctx->stream, X, Y, nm, nx, ny, nz, width, rows,
+                               part);
+        };
+        const std::integral_constant<int, 1> one{};
+        const std::integral_constant<int, 2> two{};
+        if (swap) cout == 1 ? run(one, std::true_type{}) : run(two, std::true_type{});
+        else cin == 1 ? run(one, std::false_type{}) : run(two, std::false_type{});
     }
     DAGE_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(sum_blocks_kernel, dim3((len + 31) / 32), dim3(256), 0, ctx->stream, part,

@@ -67,3 +67,9 @@ def check(ctx, nx, ny, nz, cin, cout):
 @pytest.mark.parametrize("cin,cout", [(16, 16), (3, 5)])
 def test_infinity_stays_with_its_taps(ctx, size, cin, cout):
     check(ctx, *size, cin, cout)
+
+
+@pytest.mark.parametrize("size", SIZES["few"])
+@pytest.mark.parametrize("cin,cout", [(2, 16), (1, 16), (16, 1), (16, 2), (7, 2), (1, 1)])
+def test_infinity_few_channels(ctx, size, cin, cout):
+    check(ctx, *size, cin, cout)

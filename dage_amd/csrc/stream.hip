@@ -122,7 +122,9 @@ __global__ void __launch_bounds__(256) pack_blocks_kernel(const double *f, long 
 
 // Wavefronts per SIMD of stream_xy_kernel<N> and stream_z_kernel<N>: as many
 // as the accumulators, Fx and the loads in flight leave registers for.
-constexpr int xy_waves(int n) { return n <= 2 ? 4 : (n <= 5 ? 3 : (n <= 9 ? 2 : 1)); }
+constexpr int xy_waves(int n, int w) {  // blocks of w wavefronts
+    return n <= 2 ? 4 : (n <= 5 ? 3 : (n <= 9 || (n == 10 && w == 4) ? 2 : 1));
+}
 constexpr int z_waves(int n) { return n <= 6 ? 4 : (n <= 9 ? 3 : 2); }
 
 struct StreamXY {
@@ -140,7 +142,7 @@ struct StreamXY {
 
 template <int N, int W, bool RING>
 __global__ void __launch_bounds__(64 * W)
-    __attribute__((amdgpu_waves_per_eu(xy_waves(N))))
+    __attribute__((amdgpu_waves_per_eu(xy_waves(N, W))))
     stream_xy_kernel(StreamXY a) {
     constexpr int HB = (N - 1) / 2;
     constexpr int FT = 128 * N;                       // 16-byte pieces of an Fy panel
@@ -217,6 +219,7 @@ __global__ void __launch_bounds__(64 * W)
         return left >= 2 ? 0u : (left == 1 ? 0u - 8u : kOutside);
     };
     const unsigned tail0 = tail_delta(0), tail1 = tail_delta(1);
+    const bool odd0 = tail0 == 0u - 8u, odd1 = tail1 == 0u - 8u;
     auto load_x = [&](int q, unsigned xm) {
         const unsigned skip = (xm >> (2 * q)) & 3u ? 0u : kOutside;
         const int d = 2 * (q % D);
@@ -276,6 +279,12 @@ __global__ void __launch_bounds__(64 * W)
         for (int q = 0; q < NQ; ++q) {
             if (q < N) {
                 const int d = 2 * (q % D);
+                if (__builtin_expect(q == qend, 0)) {
+                    // the point before the last counts in its own pair; here
+                    // it would turn an infinity into a NaN
+                    x[d][0] = odd0 ? 0.0 : x[d][0];
+                    x[d + 1][0] = odd1 ? 0.0 : x[d + 1][0];
+                }
 #pragma unroll
                 for (int c = 0; c < 2; ++c)
                     if (__builtin_expect((xm >> (2 * q + c)) & 1u, 1)) {
@@ -686,7 +695,7 @@ int stream_run(const ApplyMats &m, int t0, int t1, int B, int *tiles) {
     while (end < t1 && xy_tiles(m, end) != 0) ++end;
     // rounds of the card's wavefront slots that n t-points fill
     const double waves = (double)((m.dout[0] + 15) / 16) * m.din[2] * B;
-    auto rounds = [&](int n, int c) { return n * waves / (1024.0 * xy_waves(std::abs(c))); };
+    auto rounds = [&](int n, int c) { return n * waves / (1024.0 * xy_waves(std::abs(c), 2)); };
     auto wider = [](int a, int b) { return a < 0 || b < 0 ? std::min(a, b) : std::max(a, b); };
     int e = t0, code = 0;
     while (e < end) {

@@ -72,3 +72,35 @@ def test_streamed_passes(ctx, monkeypatch, case):
     ref = O.transform_cube(F[0], F[1].transpose(1, 0, 2).copy("F"), F[2].transpose(1, 0, 2).copy("F"),
                            w, 0.0, x, add_coda=False)
     assert rel_maxdiff(got["1"], ref) < 1e-10
+
+
+@pytest.mark.parametrize("n,band", [(5, 5), (17, 17), (31, 31), (33, 33), (95, 95), (97, 12), (209, 20)])
+def test_infinity_on_odd_axes(ctx, n, band):
+    """Positive matrices and inputs, one infinity near the end of the x axis:
+    every output it reaches is +inf, not NaN (an odd axis ends in the middle
+    of the x product's pairs of points)."""
+    ax, short = O.Axis(0.0, np.full(n - 1, 0.2), 2), O.Axis(0.0, np.full(4, 0.2), 2)
+    q = dage_amd.GaussQuad(nlin=3, nlog=0, tlin=2.0, tlog=2.0)
+    T = q.get_npoints()
+    rng = np.random.default_rng(n)
+
+    def matrix(m):
+        i = np.arange(m)
+        return np.where(np.abs(i[:, None] - i) <= band, 1.0, 0.0)[:, :, None] * rng.uniform(0.5, 1.0, (m, m, T))
+
+    Fx, Fy, Fz = matrix(n), matrix(n), matrix(5)
+    g = dage_amd.Grid3D(ctx, [0.0] * 3, [ax.steps, ax.steps, short.steps], 2)
+    op = dage_amd.Coulomb3D(ctx, g, g, q, coda=False)
+    op.set_matrices(np.asfortranarray(Fx), np.asfortranarray(Fy), np.asfortranarray(Fz))
+    for x, y, z in ((n - 2, 0, 1), (n - 1, n // 2, 2), (n - 3, n - 1, 0), (0, n - 2, 4)):
+        cube = rng.uniform(0.5, 1.0, (n, n, 5))
+        cube[x, y, z] = np.inf
+        a, b = dage_amd.DeviceCube(ctx, cube.shape, cube), dage_amd.DeviceCube(ctx, cube.shape)
+        ctx.profile(True)
+        op.transform_cuda_cube(a, b)
+        assert ctx.profile_query("gemm_f64_xymode")[1] > 0
+        ctx.profile(False)
+        out = b.download()
+        reach = (Fx[:, x, 0] > 0)[:, None, None] & (Fy[y, :, 0] > 0)[None, :, None] & np.ones(5, bool)
+        assert np.all(np.isposinf(out[reach])), (x, y, z)
+    op.close()

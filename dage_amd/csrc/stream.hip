@@ -659,7 +659,9 @@ static int xy_tiles(const ApplyMats &m, int t) {
     const bool square = m.din[0] == m.dout[0] && m.din[1] == m.dout[1] && m.dout[1] <= 1024;
     const int ring = square ? 2 * std::max(1, m.hb[t]) + 1 : kMaxTiles + 1;
     if (ring <= kMaxTiles && ring < full) return ring;
-    return full <= kMaxTiles ? -std::max(full, 2) : 0;
+    // four tiles run on five: a kernel of four spilled at three wavefronts per
+    // SIMD and is slower at two (57^3: 101 and 86 us, 74 on five)
+    return full <= kMaxTiles ? -std::max(full == 4 ? 5 : full, 2) : 0;
 }
 
 // Whether the streamed passes take this operator's sizes at all.
@@ -739,7 +741,6 @@ int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, dou
     case 13: rc = launch_xy_n<13, true>(a, B, s); break;
     case -2: rc = launch_xy_n<2, false>(a, B, s); break;
     case -3: rc = launch_xy_n<3, false>(a, B, s); break;
-    case -4: rc = launch_xy_n<4, false>(a, B, s); break;
     case -5: rc = launch_xy_n<5, false>(a, B, s); break;
     case -6: rc = launch_xy_n<6, false>(a, B, s); break;
     case -7: rc = launch_xy_n<7, false>(a, B, s); break;

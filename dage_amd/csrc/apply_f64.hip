@@ -556,7 +556,9 @@ bool tgroup_x() {
 // half the workspace at one t-point, so larger cubes fit a limited scratch.
 struct Plan {
     int tchunk;
-    int splits;
+    int splits;   // partials of the z products: the larger of the passes' splits
+    int zsplits;  // splits of the streamed z pass and of the separate one
+    int gsplits;
     bool no_v;
     size_t v_elems, u_elems, p_elems;
 };
@@ -570,21 +572,28 @@ Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
     if (const char *e = std::getenv("DAGE_APPLY_WORKSPACE_MB")) budget = (size_t)atol(e) << 20;
     const size_t total_cap = 64ull << 30;  // and for all B right-hand sides together
     const char *fu = std::getenv("DAGE_APPLY_FUSED");
-    const bool no_v = fu && fu[0] == '1' && streams_all(m);
+    const bool no_v = fu && fu[0] == '1' && stream_count(m, 0, m.ntp) == m.ntp;
     const size_t vt = no_v ? 0 : (size_t)(nxo * nyi * nzi);
     const size_t per_t = 8ull * (vt + (size_t)(nxo * nyo * nzi));
     const long M3 = nxo * nyo;
     const int mtiles = (int)((M3 + 64 * kMW - 1) / (64 * kMW));
     const int nb = pick_nb((int)nzo);
     const int ntiles = (int)((nzo + 16 * nb - 1) / (16 * nb));
+    // The t-points between the low-rank head and the banded tail run streamed
+    // or separately, and each z pass has its own rule: the streamed one's in
+    // z_splits; the separate one aims at 1024 blocks (121 x 121 x 33 points from
+    // 241 x 241 x 65: 867 us at z_splits' splits, 809 at its own).
+    const int tlo = lowrank_pays(m, B) ? m.lr->t1 : 0, thi = band_pays(m, B) ? m.band_t0 : m.ntp;
+    const int nstream = no_v ? m.ntp : stream_count(m, tlo, thi);
+    const bool streamed = nstream > 0, separate = !no_v && nstream < thi - tlo;
     auto fill = [&](int tchunk) {
         Plan p;
         p.tchunk = tchunk;
         p.no_v = no_v;
-        const long K3 = nzi * p.tchunk;
-        int splits = m.fxp ? z_splits(m, B)
-                           : std::max(1, (1024 + mtiles * ntiles * B - 1) / (mtiles * ntiles * B));
-        splits = (int)std::min<long>(splits, std::max<long>(1, K3 / 64));
+        const int kmax = (int)std::max<long>(1, nzi * p.tchunk / 64);
+        p.zsplits = streamed ? std::min(z_splits(m, B), kmax) : 1;
+        p.gsplits = separate ? std::min(std::max(1, (1024 + mtiles * ntiles * B - 1) / (mtiles * ntiles * B)), kmax) : 1;
+        const int splits = std::max(p.zsplits, p.gsplits);
         p.splits = splits;
         p.v_elems = vt * p.tchunk * B;
         p.u_elems = (size_t)nxo * nyo * nzi * p.tchunk * B;
@@ -1052,7 +1061,7 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
                 tc += r;
             }
             if (tc > 0) {
-                const int splits = plan.splits;
+                const int splits = std::min(plan.zsplits, plan.splits);
                 DAGE_TRY(stream_z(ctx, m, V, Ut, Ut * tstream, t0, direct ? out : P,
                                   slab * plan.splits, slab, splits, pinit, t0, tc, B, nm_z));
                 pinit = std::max(pinit, splits);
@@ -1129,7 +1138,8 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
 
         // pass 3, batch (split, b): P_{b,s}((xo,yo), zo) (+)= U_b((xo,yo), k) . Gz(k, zo)
         const int K3 = (int)(nzi * tc);
-        const int ks = (K3 + plan.splits - 1) / plan.splits;
+        const int gs = std::min(plan.gsplits, plan.splits);
+        const int ks = (K3 + gs - 1) / gs;
         const int splits = (K3 + ks - 1) / ks;
         Gemm g3{};
         g3.A = U;

@@ -427,7 +427,8 @@ void stream_mats(dage_operator op, ApplyMats *m);
 // Number of leading t-points of [t0, t1) one stream_xy call of B right-hand
 // sides takes (0: t0 cannot be streamed) and its kernel's tiles.
 int stream_run(const ApplyMats &m, int t0, int t1, int B, int *tiles);
-bool streams_all(const ApplyMats &m);
+// Number of the t-points of [t0, t1) whose x and y passes can run streamed
+int stream_count(const ApplyMats &m, int t0, int t1);
 int z_splits(const ApplyMats &m, int B);
 // U_{b,t} (at U + b*Ub + (t - tu)*Ut) = w_{b,t} (x and y products of in_b)
 int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, double *U, long Ut,

@@ -675,10 +675,11 @@ static bool streams(const ApplyMats &m) {
     return !(e && e[0] == '0');
 }
 
-bool streams_all(const ApplyMats &m) {
-    for (int t = 0; t < m.ntp; ++t)
-        if (!streams(m) || xy_tiles(m, t) == 0) return false;
-    return true;
+int stream_count(const ApplyMats &m, int t0, int t1) {
+    int n = 0;
+    if (streams(m))
+        for (int t = t0; t < t1; ++t) n += xy_tiles(m, t) != 0;
+    return n;
 }
 
 // Rounds of the card's wavefront slots below which a launch is not worth its

@@ -6,12 +6,15 @@ Both paths sum the same products (the flushed matrices' zeros are skipped by
 either), in another order: at every point they differ by at most
 2 (nx + ny + nz + T + 3) 2^-53 times the sum of the products' magnitudes.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import dage_amd
 import oracle as O
 from _helpers import rel_maxdiff
+from dage_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 
@@ -103,4 +106,23 @@ def test_infinity_on_odd_axes(ctx, n, band):
         out = b.download()
         reach = (Fx[:, x, 0] > 0)[:, None, None] & (Fy[y, :, 0] > 0)[None, :, None] & np.ones(5, bool)
         assert np.all(np.isposinf(out[reach])), (x, y, z)
+    op.close()
+
+
+def test_separate_z_pass_keeps_its_split_rule(ctx, monkeypatch):
+    """Different grids with an axis above 208 points run the separate passes,
+    whose z pass splits its sum for about 1024 blocks: the workspace holds
+    that many partials, not the streamed pass's."""
+    monkeypatch.setenv("DAGE_APPLY_TCHUNK", "24")
+    nin, nout = (241, 241, 65), (121, 121, 33)
+    gin, gout = (dage_amd.Grid3D(ctx, [0.0] * 3, [np.full((n - 1) // 4, s) for n in shape], 5)
+                 for shape, s in ((nin, 0.4), (nout, 0.8)))
+    q = dage_amd.GaussQuad(nlin=12, nlog=12, tlin=2.0, tlog=300.0)
+    op = dage_amd.Coulomb3D(ctx, gin, gout, q, coda=False)
+    size = ctypes.c_size_t()
+    call("dage_operator_workspace_bytes", op.handle, ctypes.byref(size))
+    per_t = nout[0] * (nin[1] + nout[1]) * nin[2]
+    tiles = (nout[0] * nout[1] + 63) // 64  # one 48-column tile in z
+    splits = (1024 + tiles - 1) // tiles
+    assert splits == 5 and size.value == 8 * (24 * per_t + splits * nout[0] * nout[1] * nout[2])
     op.close()

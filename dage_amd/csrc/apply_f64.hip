@@ -560,6 +560,7 @@ struct Plan {
     int zsplits;  // splits of the streamed z pass and of the separate one
     int gsplits;
     bool no_v;
+    bool streamed;  // the t-points that can run streamed do
     size_t v_elems, u_elems, p_elems;
 };
 
@@ -584,12 +585,13 @@ Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
     // z_splits; the separate one aims at 1024 blocks (121 x 121 x 33 points from
     // 241 x 241 x 65: 867 us at z_splits' splits, 809 at its own).
     const int tlo = lowrank_pays(m, B) ? m.lr->t1 : 0, thi = band_pays(m, B) ? m.band_t0 : m.ntp;
-    const int nstream = no_v ? m.ntp : stream_count(m, tlo, thi);
-    const bool streamed = nstream > 0, separate = !no_v && nstream < thi - tlo;
+    const bool streamed = no_v || stream_pays(m, tlo, thi, B);
+    const bool separate = !no_v && !(streamed && stream_count(m, tlo, thi) == thi - tlo);
     auto fill = [&](int tchunk) {
         Plan p;
         p.tchunk = tchunk;
         p.no_v = no_v;
+        p.streamed = streamed;
         const int kmax = (int)std::max<long>(1, nzi * p.tchunk / 64);
         p.zsplits = streamed ? std::min(z_splits(m, B), kmax) : 1;
         p.gsplits = separate ? std::min(std::max(1, (1024 + mtiles * ntiles * B - 1) / (mtiles * ntiles * B)), kmax) : 1;
@@ -1053,7 +1055,7 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
                             ? tcmax : (int)((plan.v_elems + plan.u_elems) / ((size_t)Ut * B));
     for (int t0 = tlr; t0 < T;) {
         const bool banded = t0 >= tb;
-        if (!banded) {
+        if (!banded && plan.streamed) {
             const int tend = std::min(tb, t0 + tstream);
             int tc = 0, tiles = 0;
             while (const int r = stream_run(m, t0 + tc, tend, B, &tiles)) {
@@ -1070,7 +1072,7 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
             }
         }
         int tc = std::min(tcmax, (banded ? T : tb) - t0), tiles = 0;
-        if (!banded)  // up to the next t-point that can be streamed
+        if (!banded && plan.streamed)  // up to the next t-point that can be streamed
             for (int e = 1; e < tc; ++e)
                 if (stream_run(m, t0 + e, t0 + e + 1, B, &tiles) > 0) tc = e;
         // pass 1, batch (t, b): V_{b,t}((yi,zi), xo) = in_b((yi,zi), xi) . Fx_t^T(xi, xo)

@@ -244,6 +244,7 @@ struct dage_operator_s {
     double *d_pack = nullptr;
     size_t pack_off[3] = {0, 0, 0};
     std::vector<int> tile_hb;
+    std::vector<int2> tile_blocks;  // 16 x 16 blocks with entries of Fx_t (x) and Fy_t (y)
     // d_steps: the z pass's lists of panels, for each group of output tiles,
     // each number of splits S and split s of it from z_off[.] on; z_t: their t
     int4 *d_steps = nullptr;
@@ -305,11 +306,13 @@ struct ApplyMats {
     // pitch tiling (pitch[p] > 0): tile masks, same row order, bit j = tile j
     const uint64_t *tmask[3] = {nullptr, nullptr, nullptr};
     int pitch[3] = {0, 0, 0}, nbp[3] = {0, 0, 0};
-    // streamed passes (dage_operator_s::d_pack, d_ranges, tile_hb; null: none)
+    // streamed passes (dage_operator_s::d_pack, d_ranges, tile_hb, tile_blocks; null:
+    // none)
     const double *fxp = nullptr, *fyp = nullptr, *fzp = nullptr;
     const int2 *xr = nullptr, *yr = nullptr;
     const int *hb = nullptr, *z_off = nullptr, *z_t = nullptr;
     const int4 *zsteps = nullptr;
+    const int2 *blocks = nullptr;
     // banded y/z passes for t >= band_t0 (see dage_operator_s)
     const double *band_y = nullptr, *band_z = nullptr, *band_x = nullptr;
     int band_t0 = 0, band_mode = 1;
@@ -429,6 +432,8 @@ void stream_mats(dage_operator op, ApplyMats *m);
 int stream_run(const ApplyMats &m, int t0, int t1, int B, int *tiles);
 // Number of the t-points of [t0, t1) whose x and y passes can run streamed
 int stream_count(const ApplyMats &m, int t0, int t1);
+// ... and whether they do in a call of B right-hand sides
+bool stream_pays(const ApplyMats &m, int t0, int t1, int B);
 int z_splits(const ApplyMats &m, int B);
 // U_{b,t} (at U + b*Ub + (t - tu)*Ut) = w_{b,t} (x and y products of in_b)
 int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, double *U, long Ut,

@@ -478,18 +478,20 @@ int launch_xy_w(const StreamXY &a0, int B, hipStream_t s) {
     return DAGE_OK;
 }
 
+// Wavefronts per block of stream_xy_kernel<N> for nxt x tiles: the group size
+// that leaves the fewest idle, of those that fill the SIMDs (3 per block only
+// with 3 per SIMD: with 2, two of a CU's eight slots stay empty; 385^3, 25 x
+// tiles, N = 7 and 9: 12.0 -> 10.0 ms with 2 instead of 3)
+int group_size(int N, int nxt) {
+    auto idle = [&](int w) { return (nxt + w - 1) / w * w - nxt; };
+    const int w = N >= 3 && N <= 5 ? 3 : 2;
+    return idle(w) < idle(4) ? w : 4;
+}
+
 template <int N, bool RING>
 int launch_xy_n(const StreamXY &a, int B, hipStream_t s) {
-    // Wavefronts per block: the group size that leaves the fewest idle, of
-    // those that fill the SIMDs (3 per block only with 3 per SIMD: with 2,
-    // two of a CU's eight slots stay empty; 385^3, 25 x tiles, N = 7 and 9:
-    // 12.0 -> 10.0 ms with 2 instead of 3)
-    auto idle = [&](int w) { return (a.nxt + w - 1) / w * w - a.nxt; };
-    if constexpr (N >= 3 && N <= 5) {
-        if (idle(3) < idle(4)) return launch_xy_w<N, 3, RING>(a, B, s);
-        return launch_xy_w<N, 4, RING>(a, B, s);
-    }
-    if (idle(2) < idle(4)) return launch_xy_w<N, 2, RING>(a, B, s);
+    constexpr int w = N >= 3 && N <= 5 ? 3 : 2;
+    if (group_size(N, a.nxt) == w) return launch_xy_w<N, w, RING>(a, B, s);
     return launch_xy_w<N, 4, RING>(a, B, s);
 }
 
@@ -555,13 +557,18 @@ int build_stream(dage_operator op, const std::vector<int> &span) {
     }
     std::vector<int2> rg(ranges);
     op->tile_hb.assign(T, 0);
+    op->tile_blocks.assign(T, make_int2(0, 0));
     int2 *rp = rg.data();
     for (int a = 0; a < 3; ++a) {
         for (long t = 0; t < T; ++t) {
             int2 *r = rp + t * nt[a];
             const int hb = tile_ranges(span.data(), row[a] + t * op->din[a], op->din[a],
                                        op->dout[a], r);
-            if (a < 2) op->tile_hb[t] = std::max(op->tile_hb[t], hb);
+            if (a == 2) continue;
+            op->tile_hb[t] = std::max(op->tile_hb[t], hb);
+            int n = 0;  // 16 x 16 blocks
+            for (long j = 0; j < nt[a]; ++j) n += r[j].x < r[j].y ? (r[j].y + 3) / 4 - r[j].x / 4 : 0;
+            (a == 0 ? op->tile_blocks[t].x : op->tile_blocks[t].y) = n;
         }
         rp += T * nt[a];
     }
@@ -645,6 +652,7 @@ void stream_mats(dage_operator op, ApplyMats *m) {
     m->fyp = op->d_pack + op->pack_off[1];
     m->fzp = op->d_pack + op->pack_off[2];
     m->hb = op->tile_hb.data();
+    m->blocks = op->tile_blocks.data();
     m->zsteps = op->d_steps;
     m->z_off = op->z_off.data();
     m->z_t = op->z_t.data();
@@ -664,15 +672,20 @@ static int xy_tiles(const ApplyMats &m, int t) {
     return full <= kMaxTiles ? -std::max(full == 4 ? 5 : full, 2) : 0;
 }
 
+// DAGE_APPLY_STREAM (read at every call): 0 never streams, 1 wherever it can
+// (comparison runs, tests), else where it is faster (stream_pays).
+static char stream_mode() {
+    const char *e = std::getenv("DAGE_APPLY_STREAM");
+    return e ? e[0] : 0;
+}
+
 // Whether the streamed passes take this operator's sizes at all.
-// DAGE_APPLY_STREAM=0 turns them off (comparison runs; read at every call).
 static bool streams(const ApplyMats &m) {
     if (!m.xr || !m.fxp) return false;
     // byte offsets within a plane of the cubes and 16 planes of U below 2^31
     if ((long)m.din[0] * (m.din[1] + 32) >= (1L << 28)) return false;
     if ((long)m.dout[0] * (m.dout[1] + 16) >= (1L << 24)) return false;
-    const char *e = std::getenv("DAGE_APPLY_STREAM");
-    return !(e && e[0] == '0');
+    return stream_mode() != '0';
 }
 
 int stream_count(const ApplyMats &m, int t0, int t1) {
@@ -715,6 +728,69 @@ int stream_run(const ApplyMats &m, int t0, int t1, int B, int *tiles) {
     }
     *tiles = code;
     return e - t0;
+}
+
+// Estimated us of the x and y products of [t0, t1) on the streamed and on the
+// separate passes.  Both grow with the 16 x 16 blocks that the matrices need,
+// but the streamed kernel pads the x axis to whole tiles and groups of
+// wavefronts and loads its whole window for every wavefront and panel, while
+// the separate passes pad only the flattened rows: thin boxes are slower
+// streamed (9 x 213 x 145 points: 579 against 172 us, 41 x 401 x 41: 651
+// against 394).  The coefficients are least-squares fits to the measured times
+// of 1380 boxes, pairs of grids and batches with axes of 5 to 421 points
+// (standard deviation 14 % streamed, 17 % separate).  Streaming needs a margin of
+// 5 %: with it the call is slower than without in under 1 % of them by more
+// than 5 %, and of the boxes with sides within 1.6 of each other all but one of
+// 236 stream (they gain 1.1 to 1.8).
+constexpr double kLaunch = 5.2;   // a launch
+constexpr double kStart = 2.1;    // a wavefront's Fx window and first loads
+constexpr double kPanel = 0.81;   // a panel
+constexpr double kLoad = 0.116;   // a block of a wavefront's window, per panel
+constexpr double kBlock = 0.111;  // a block's products
+constexpr double kBesides = 10.0; // the separate passes' launches beside
+constexpr double kSepLaunch = 11.3;       // the two passes
+constexpr double kSepStep = 1.06;         // a panel of either sum
+constexpr double kSepBlock = 1.41e-3;     // a block's products of 64 rows
+constexpr double kSepPanel = 3.8e-4;      // the rows' panels
+constexpr double kMargin = 1.05;
+
+static void xy_costs(const ApplyMats &m, int t0, int t1, int B, double *stream, double *separate) {
+    const int nxt = (m.dout[0] + 15) / 16, nxb = (m.din[0] + 15) / 16;
+    const int nyb = (m.din[1] + 15) / 16;
+    const double rx = (m.din[1] * (long)m.din[2] + 63) / 64 * (double)B;
+    const double ry = (m.dout[0] * (long)m.din[2] + 63) / 64 * (double)B;
+    bool rest = false;  // t-points that run separately in any case
+    *stream = *separate = 0.0;
+    for (int t = t0, r, code = 0; t < t1; t += r) {
+        r = stream_run(m, t, t1, B, &code);
+        if (r == 0) {
+            rest = true;
+            r = 1;
+            continue;
+        }
+        double x = 0.0, y = 0.0;
+        for (int e = t; e < t + r; ++e) x += m.blocks[e].x, y += m.blocks[e].y;
+        *separate += kSepBlock * (rx * x + ry * y) + kSepPanel * (rx * x / nxb + ry * y / nyb);
+        // wavefronts per SIMD, those of them with work, rounds of the card
+        const int N = std::abs(code), W = group_size(N, nxt), groups = (nxt + W - 1) / W;
+        const double w = xy_waves(N, W), act = w * nxt / (groups * W);
+        const double rounds = (double)groups * W * r * m.din[2] * B / (1024.0 * w);
+        const double blk = kBlock * (x / nxt + y / nyb) / r;  // of a wavefront's panel
+        const double one = kPanel + kLoad * N + blk;
+        const double round = kStart + nyb * std::max(one, kLoad * N * w + blk * act);
+        *stream += kLaunch + std::max(0.5 * kStart + nyb * one, rounds * round);
+    }
+    if (rest) *stream += kBesides;
+    else *separate += kSepLaunch + kSepStep * (nxb + nyb);
+}
+
+// Whether the t-points of [t0, t1) that can run streamed do.
+bool stream_pays(const ApplyMats &m, int t0, int t1, int B) {
+    if (stream_count(m, t0, t1) == 0) return false;
+    if (stream_mode() == '1') return true;
+    double stream, separate;
+    xy_costs(m, t0, t1, B, &stream, &separate);
+    return kMargin * stream <= separate;
 }
 
 int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, double *U, long Ut,

@@ -78,7 +78,7 @@ def test_streamed_passes(ctx, monkeypatch, case):
 
 
 @pytest.mark.parametrize("n,band", [(5, 5), (17, 17), (31, 31), (33, 33), (95, 95), (97, 12), (209, 20)])
-def test_infinity_on_odd_axes(ctx, n, band):
+def test_infinity_on_odd_axes(ctx, monkeypatch, n, band):
     """Positive matrices and inputs, one infinity near the end of the x axis:
     every output it reaches is +inf, not NaN (an odd axis ends in the middle
     of the x product's pairs of points)."""
@@ -95,6 +95,7 @@ def test_infinity_on_odd_axes(ctx, n, band):
     g = dage_amd.Grid3D(ctx, [0.0] * 3, [ax.steps, ax.steps, short.steps], 2)
     op = dage_amd.Coulomb3D(ctx, g, g, q, coda=False)
     op.set_matrices(np.asfortranarray(Fx), np.asfortranarray(Fy), np.asfortranarray(Fz))
+    monkeypatch.setenv("DAGE_APPLY_STREAM", "1")
     for x, y, z in ((n - 2, 0, 1), (n - 1, n // 2, 2), (n - 3, n - 1, 0), (0, n - 2, 4)):
         cube = rng.uniform(0.5, 1.0, (n, n, 5))
         cube[x, y, z] = np.inf
@@ -125,4 +126,27 @@ def test_separate_z_pass_keeps_its_split_rule(ctx, monkeypatch):
     tiles = (nout[0] * nout[1] + 63) // 64  # one 48-column tile in z
     splits = (1024 + tiles - 1) // tiles
     assert splits == 5 and size.value == 8 * (24 * per_t + splits * nout[0] * nout[1] * nout[2])
+    op.close()
+
+
+@pytest.mark.parametrize("shape,streams", [((65, 65, 65), True), ((45, 57, 61), True),
+                                           ((9, 213, 145), False), ((41, 401, 41), False),
+                                           ((5, 173, 85), False)])
+def test_thin_boxes_keep_the_separate_passes(ctx, monkeypatch, shape, streams):
+    """The default route by shape; the same result as on the other route (the
+    bound of this file's header, with every |entry| at most its row's sum)."""
+    monkeypatch.delenv("DAGE_APPLY_STREAM", raising=False)
+    g = dage_amd.Grid3D(ctx, [0.0] * 3, [np.full((n - 1) // 4, 0.8) for n in shape], 5)
+    op = dage_amd.Coulomb3D(ctx, g, g, dage_amd.GaussQuad(nlin=20, nlog=20, tlin=2.0, tlog=500.0))
+    x = np.random.default_rng(7).uniform(0.0, 1.0, shape)
+    a, b = dage_amd.DeviceCube(ctx, shape, x), dage_amd.DeviceCube(ctx, shape)
+    ctx.profile(True)
+    op.transform_cuda_cube(a, b)
+    count = ctx.profile_query("gemm_f64_xymode")[1], ctx.profile_query("gemm_f64_xmode")[1]
+    ctx.profile(False)
+    assert (count[0] > 0) == streams and (count[1] > 0) == (not streams)
+    got = b.download().copy()
+    monkeypatch.setenv("DAGE_APPLY_STREAM", "0" if streams else "1")
+    op.transform_cuda_cube(a, b)
+    assert rel_maxdiff(got, b.download()) < 1e-13
     op.close()

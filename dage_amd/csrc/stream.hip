@@ -165,7 +165,9 @@ __global__ void __launch_bounds__(64 * W)
     const int slot = (int)((unsigned)(wave + blockIdx.x / (unsigned)a.groups) % (unsigned)W);
     const int it = g * W + slot;
     const bool active = it < a.nxt;
-    const int xs = RING && active ? it - HB : 0;  // first 16-point x block of the window
+    // first 16-point x block of the window; the full one ends with the axis, so
+    // that the block of the axis end is known at compile time
+    const int xs = RING ? (active ? it - HB : 0) : a.nxb - N;
     const __amdgpu_buffer_rsrc_t rin =
         buffer(a.in + (long)b * a.nin + (long)z0 * a.nxi * a.nyi,
                8u * (unsigned)a.nxi * (unsigned)a.nyi);
@@ -218,13 +220,15 @@ __global__ void __launch_bounds__(64 * W)
         const int left = (a.nxi & 15) - 8 * c - 2 * lk;  // points from the pair's first on
         return left >= 2 ? 0u : (left == 1 ? 0u - 8u : kOutside);
     };
-    const unsigned tail0 = tail_delta(0), tail1 = tail_delta(1);
+    const bool tail = !RING && qend >= 0;
+    const unsigned tail0 = RING || tail ? tail_delta(0) : 0u, tail1 = RING || tail ? tail_delta(1) : 0u;
+    auto at_end = [&](int q) { return RING ? q == qend : q == N - 1; };
     const bool odd0 = tail0 == 0u - 8u, odd1 = tail1 == 0u - 8u;
     auto load_x = [&](int q, unsigned xm) {
         const unsigned skip = (xm >> (2 * q)) & 3u ? 0u : kOutside;
         const int d = 2 * (q % D);
-        x[d] = buf_ld2(rin, (xoff + 128 * q + (q == qend ? tail0 : 0u)) | skip);
-        x[d + 1] = buf_ld2(rin, (xoff + 128 * q + 64 + (q == qend ? tail1 : 0u)) | skip);
+        x[d] = buf_ld2(rin, (xoff + 128 * q + (at_end(q) ? tail0 : 0u)) | skip);
+        x[d + 1] = buf_ld2(rin, (xoff + 128 * q + 64 + (at_end(q) ? tail1 : 0u)) | skip);
     };
     d2 rf[FW];
     // the panel's Fy blocks: all nyt of them, or the window from p - HB (the
@@ -279,7 +283,7 @@ __global__ void __launch_bounds__(64 * W)
         for (int q = 0; q < NQ; ++q) {
             if (q < N) {
                 const int d = 2 * (q % D);
-                if (__builtin_expect(q == qend, 0)) {
+                if (RING ? __builtin_expect(q == qend, 0) : q == N - 1 && tail) {
                     // the point before the last counts in its own pair; here
                     // it would turn an infinity into a NaN
                     x[d][0] = odd0 ? 0.0 : x[d][0];

@@ -245,7 +245,8 @@ int dage_ctx_create(int device, dage_ctx *out) {
         return DAGE_ERR_HIP;
     }
     ctx->stream = ctx->own_stream;
-    const int rc = scratch_address(device, &ctx->noalloc_scratch);
+    int rc = prepare_fused_kernels();
+    if (rc == DAGE_OK) rc = scratch_address(device, &ctx->noalloc_scratch);
     if (rc != DAGE_OK) {
         (void)hipStreamDestroy(ctx->own_stream);
         delete ctx;

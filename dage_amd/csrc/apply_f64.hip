@@ -388,6 +388,178 @@ __global__ void __launch_bounds__(kThreads) gemm_f64_kernel(Gemm g) {
     }
 }
 
+// Fused x and y passes for workspaces without room for V (DAGE_APPLY_FUSED=1)
+// where the streamed kernels do not fit, on axes up to 16*kMaxNT points: for
+// one (right-hand side b, t, input z-plane zi) and 64 output x points (16 per
+// wavefront),
+//   U(xo, yo) = w_t sum_yi [sum_xi Fx_t(xo,xi) in(xi,yi,zi)] Fy_t(yi,yo),
+// without the x-pass intermediate V reaching memory.  The input y axis is
+// walked in chunks of 16 points.  Per chunk a wavefront first forms the
+// 16 x 16 tile V^T(yi, xo) = in^T(yi, xi) Fx_t^T(xi, xo) on the MFMA (A = the
+// input chunk from LDS, B = Fx_t from global memory); result register r of
+// lane l then holds V(xo = l%16, yi = 4r + l/16), which is exactly the
+// A-operand element of k-step r of the y product, so the tile feeds
+//   U(xo, yo) += V(xo, yi-chunk) Fy_t(yi-chunk, yo)
+// straight from registers (B = the Fy_t chunk from LDS), one accumulator per
+// 16-point output y tile.  The k-grouping, operand roles and k order are those
+// of the separate x and y passes, and only products with a zero matrix entry
+// outside the bands are skipped, so U is bit-identical to theirs.
+//
+// The input chunk (16 columns of nxi points, contiguous in memory) and the
+// Fy_t chunk (16 rows) are staged in LDS, the next chunk's loads issued into
+// registers before the current chunk's MFMAs.  NT >= the output y tiles and
+// NT >= nxi / 16 (it also sizes the loader's registers).
+struct XYF {
+    const double *in;   // in_b(xi, yi, zi) at in + b*nin + xi + nxi*(yi + nyi*zi)
+    const double *fx;   // Fx_t(xo, xi) at fx + xo + nxo*(xi + nxi*t)
+    const double *fy;   // Fy_t(yi, yo) at fy + yi + nyi*(yo + nyo*t)
+    double *U;          // U + xo + nxo*(yo + nyo*zi) + Ut*(tl + tc*b)
+    const double *w;    // alpha = w[t0 + tl + wS*b]
+    long wS;
+    int nxi, nyi, nxo, nyo, nzi;
+    int t0, tc;
+    long nin, Ut;
+    const int2 *xr, *yr;  // k-step ranges of the x and y tiles (ApplyMats)
+    int nxt, nyt;
+    int gx;      // 64-point output x blocks
+    int ldy;     // LDS row count of the Fy chunk (16 * output y tiles)
+    int remap;
+};
+
+template <int NT>
+__global__ void __launch_bounds__(kThreads) xy_fused_kernel(XYF g) {
+    extern __shared__ double smem[];
+    double *Is = smem;                   // input chunk: (xi, yl) at yl*nxi + xi
+    double *Ys = smem + 16 * g.nxi;      // Fy chunk: (yl, yo) at yo*17 + yl
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int l16 = lane & 15, lk = lane >> 4;
+
+    // block -> (b, tl, zi, xb), xb fastest; XCD-aware as in block_coords
+    unsigned L = blockIdx.x;
+    if (g.remap) {
+        const unsigned total = gridDim.x;
+        const unsigned q = total >> 3, r = total & 7u, x = L & 7u;
+        L = x * q + min(x, r) + (L >> 3);
+    }
+    const int xb = (int)(L % (unsigned)g.gx);
+    L /= (unsigned)g.gx;
+    const int zi = (int)(L % (unsigned)g.nzi);
+    L /= (unsigned)g.nzi;
+    const int tl = (int)(L % (unsigned)g.tc);
+    const int b = (int)(L / (unsigned)g.tc);
+    const int t = g.t0 + tl;
+
+    const double *in = g.in + (long)b * g.nin + (long)zi * g.nxi * g.nyi;
+    const double *fx = g.fx + (long)t * g.nxo * g.nxi;
+    const double *fy = g.fy + (long)t * g.nyi * g.nyo;
+    const int xt = xb * 4 + wave;  // this wavefront's 16-point output x tile
+    const bool active = xt < g.nxt;
+    const int xo = xt * 16 + l16;
+    const bool xo_ok = xo < g.nxo;
+    const int2 xr = active ? g.xr[(long)t * g.nxt + xt] : make_int2(0, 0);
+    // lane j: the k-steps (4 input y points) that output y tile j needs
+    const int2 yr = lane < g.nyt ? g.yr[(long)t * g.nyt + lane] : make_int2(0, 0);
+    const double *fxl = fx + (xo_ok ? xo : 0);
+
+    // loaders: input chunk element e = tid + 256*s (contiguous in memory),
+    // Fy chunk element e: yl = e % 16, yo = e / 16
+    const int ichunk = 16 * g.nxi;
+    double ri[NT], ry[NT];
+    auto load_chunk = [&](int c) {
+        const int yc = 16 * c;
+        const int ilim = min(16, g.nyi - yc) * g.nxi;  // valid elements
+        const double *src = in + (long)yc * g.nxi;
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            const int e = tid + kThreads * s;
+            const bool ok = e < ilim;
+            const double v = src[ok ? e : 0];
+            ri[s] = ok ? v : 0.0;
+        }
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            const int e = tid + kThreads * s;
+            const int yl = e & 15, yo = e >> 4;
+            const bool ok = yo < g.nyo && yc + yl < g.nyi;
+            const double v = fy[ok ? (long)(yc + yl) + (long)g.nyi * yo : 0];
+            ry[s] = ok ? v : 0.0;
+        }
+    };
+    auto store_chunk = [&]() {
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            const int e = tid + kThreads * s;
+            if (e < ichunk) Is[e] = ri[s];
+        }
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            const int e = tid + kThreads * s;
+            const int yl = e & 15, yo = e >> 4;
+            if (yo < g.ldy) Ys[yo * 17 + yl] = ry[s];
+        }
+    };
+
+    d4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = d4{0.0, 0.0, 0.0, 0.0};
+
+    const int nchunks = (g.nyi + 15) / 16;
+    load_chunk(0);
+    for (int c = 0; c < nchunks; ++c) {
+        store_chunk();
+        __syncthreads();
+        if (c + 1 < nchunks) load_chunk(c + 1);
+        unsigned long long need[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) need[s] = __ballot(4 * c + s >= yr.x && 4 * c + s < yr.y);
+        if (active && (need[0] | need[1] | need[2] | need[3]) && xr.x < xr.y) {
+            // x part: V^T(yi, xo) over the k-steps of this tile's band
+            d4 v = d4{0.0, 0.0, 0.0, 0.0};
+            const double *ia = Is + l16 * g.nxi;
+            for (int s0 = xr.x; s0 < xr.y; s0 += 8) {
+                double fa[8], fb[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int xi = 4 * (s0 + u) + lk;
+                    const bool ok = s0 + u < xr.y && xi < g.nxi;
+                    const double bv = fxl[ok && xo_ok ? (long)g.nxo * xi : 0];
+                    fb[u] = ok && xo_ok ? bv : 0.0;
+                    fa[u] = ok ? ia[ok ? xi : 0] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (s0 + u < xr.y) v = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u], fb[u], v, 0, 0, 0);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    if ((need[s] >> j) & 1) {
+                        const double bv = Ys[(16 * j + l16) * 17 + 4 * s + lk];
+                        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s], bv, acc[j], 0, 0, 0);
+                    }
+            }
+        }
+        __syncthreads();
+    }
+    if (!active) return;
+    // Register r of lane l holds U(xo = xt*16 + 4r + l/16, yo = 16j + l%16).
+    const double alpha = g.w[g.t0 + tl + g.wS * b];
+    double *U = g.U + (long)zi * g.nxo * g.nyo + g.Ut * ((long)tl + (long)g.tc * b);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int yo = 16 * j + l16;
+        if (yo >= g.nyo) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int x = xt * 16 + 4 * r + lk;
+            if (x < g.nxo) U[x + (long)g.nxo * yo] = alpha * acc[j][r];
+        }
+    }
+}
+
 // Fz (nzi, nzo, T) -> Gz((zi + nzi*t), zo)
 __global__ void __launch_bounds__(256) relayout_fz_kernel(const double *fz, double *gz, int nzi,
                                                           int nzo, int T) {
@@ -550,10 +722,71 @@ bool tgroup_x() {
     return !(e && e[0] == '0');
 }
 
+constexpr int kMaxNT = 28;
+
+bool fused_wanted() {
+    const char *e = std::getenv("DAGE_APPLY_FUSED");
+    return e && e[0] == '1';
+}
+
+// The fused kernel's NT where an apply without V cannot stream, else 0: it is
+// 1.5 (97^3) to 4.4 (385^3) times slower than the separate passes, since each
+// wavefront's x product is one chain of MFMAs fed by global loads of Fx_t.
+int fused_nt(const ApplyMats &m) {
+    if (!fused_wanted() || !m.xr || stream_count(m, 0, m.ntp) == m.ntp) return 0;
+    const int need = std::max((m.dout[1] + 15) / 16, (m.din[0] + 15) / 16);
+    return need > kMaxNT ? 0 : (need + 3) / 4 * 4;
+}
+
+// Largest dynamic LDS of the fused pass: 16 input columns of up to 16*kMaxNT
+// points and 16*kMaxNT Fy rows of 17 doubles.
+constexpr size_t kFusedMaxLds = 8 * (16 * 16 * kMaxNT + 17 * 16 * kMaxNT);
+
+template <int NT>
+int set_xy_attr() {
+    DAGE_HIP_CHECK(hipFuncSetAttribute((const void *)xy_fused_kernel<NT>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)kFusedMaxLds));
+    return DAGE_OK;
+}
+
+template <int NT>
+int launch_xy_t(const XYF &g, unsigned blocks, size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL(xy_fused_kernel<NT>, dim3(blocks), dim3(kThreads), lds, s, g);
+    DAGE_HIP_CHECK(hipGetLastError());
+    return DAGE_OK;
+}
+
+int launch_xy(dage_ctx ctx, int nt, const XYF &g, int B, const char *name) {
+    const long blocks = (long)g.gx * g.nzi * g.tc * B;
+    DAGE_REQUIRE(blocks > 0 && blocks < (1L << 31), DAGE_ERR_ARG,
+                 "fused pass of %ld blocks does not fit one launch", blocks);
+    DAGE_REQUIRE(16 * nt >= g.ldy && 16 * nt >= g.nxi, DAGE_ERR_STATE,
+                 "fused pass tile %d too small", nt);
+    const size_t lds = 8 * (16 * (size_t)g.nxi + 17 * (size_t)g.ldy);
+    hipEvent_t ev;
+    prof_begin(ctx, name, &ev);
+    int rc;
+    const unsigned nb = (unsigned)blocks;
+    switch (nt) {
+    case 4: rc = launch_xy_t<4>(g, nb, lds, ctx->stream); break;
+    case 8: rc = launch_xy_t<8>(g, nb, lds, ctx->stream); break;
+    case 12: rc = launch_xy_t<12>(g, nb, lds, ctx->stream); break;
+    case 16: rc = launch_xy_t<16>(g, nb, lds, ctx->stream); break;
+    case 20: rc = launch_xy_t<20>(g, nb, lds, ctx->stream); break;
+    case 24: rc = launch_xy_t<24>(g, nb, lds, ctx->stream); break;
+    case 28: rc = launch_xy_t<28>(g, nb, lds, ctx->stream); break;
+    default: DAGE_REQUIRE(false, DAGE_ERR_STATE, "no fused pass for tile %d", nt);
+    }
+    prof_end(ctx, name, ev);
+    return rc;
+}
+
 // Workspace layout: V | U | P (split-K partials); the streamed passes, which
 // have no V, use V | U as one U.  DAGE_APPLY_FUSED=1 plans without V (and
-// without the banded and low-rank t-points) where every t-point streams:
-// half the workspace at one t-point, so larger cubes fit a limited scratch.
+// without the banded and low-rank t-points) where every t-point streams or the
+// fused kernel fits: half the workspace at one t-point, so larger cubes fit a
+// limited scratch.
 struct Plan {
     int tchunk;
     int splits;   // partials of the z products: the larger of the passes' splits
@@ -561,6 +794,7 @@ struct Plan {
     int gsplits;
     bool no_v;
     bool streamed;  // the t-points that can run streamed do
+    int fused;      // the fused kernel's NT (0: not used)
     size_t v_elems, u_elems, p_elems;
 };
 
@@ -572,8 +806,8 @@ Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
     size_t budget = 4ull << 30;  // bytes for V + U per right-hand side
     if (const char *e = std::getenv("DAGE_APPLY_WORKSPACE_MB")) budget = (size_t)atol(e) << 20;
     const size_t total_cap = 64ull << 30;  // and for all B right-hand sides together
-    const char *fu = std::getenv("DAGE_APPLY_FUSED");
-    const bool no_v = fu && fu[0] == '1' && stream_count(m, 0, m.ntp) == m.ntp;
+    const int nt = fused_nt(m);
+    const bool no_v = nt > 0 || (fused_wanted() && stream_count(m, 0, m.ntp) == m.ntp);
     const size_t vt = no_v ? 0 : (size_t)(nxo * nyi * nzi);
     const size_t per_t = 8ull * (vt + (size_t)(nxo * nyo * nzi));
     const long M3 = nxo * nyo;
@@ -585,13 +819,14 @@ Plan make_plan(const ApplyMats &m, int B = 1, size_t cap = 0) {
     // z_splits; the separate one aims at 1024 blocks (121 x 121 x 33 points from
     // 241 x 241 x 65: 867 us at z_splits' splits, 809 at its own).
     const int tlo = lowrank_pays(m, B) ? m.lr->t1 : 0, thi = band_pays(m, B) ? m.band_t0 : m.ntp;
-    const bool streamed = no_v || stream_pays(m, tlo, thi, B);
-    const bool separate = !no_v && !(streamed && stream_count(m, tlo, thi) == thi - tlo);
+    const bool streamed = no_v ? nt == 0 : stream_pays(m, tlo, thi, B);
+    const bool separate = no_v ? nt > 0 : !(streamed && stream_count(m, tlo, thi) == thi - tlo);
     auto fill = [&](int tchunk) {
         Plan p;
         p.tchunk = tchunk;
         p.no_v = no_v;
         p.streamed = streamed;
+        p.fused = nt;
         const int kmax = (int)std::max<long>(1, nzi * p.tchunk / 64);
         p.zsplits = streamed ? std::min(z_splits(m, B), kmax) : 1;
         p.gsplits = separate ? std::min(std::max(1, (1024 + mtiles * ntiles * B - 1) / (mtiles * ntiles * B)), kmax) : 1;
@@ -958,6 +1193,17 @@ ApplyMats operator_mats(dage_operator op) {
     return m;
 }
 
+int prepare_fused_kernels() {
+    DAGE_TRY(set_xy_attr<4>());
+    DAGE_TRY(set_xy_attr<8>());
+    DAGE_TRY(set_xy_attr<12>());
+    DAGE_TRY(set_xy_attr<16>());
+    DAGE_TRY(set_xy_attr<20>());
+    DAGE_TRY(set_xy_attr<24>());
+    DAGE_TRY(set_xy_attr<28>());
+    return DAGE_OK;
+}
+
 int apply_f64_workspace(dage_operator op, size_t *bytes) {
     const Plan p = make_plan(operator_mats(op));
     *bytes = 8 * (p.v_elems + p.u_elems + p.p_elems);
@@ -1021,6 +1267,7 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
     // event names (profiling): batched right-hand sides with their own
     // weights (the batch graph) apart from single applies
     const bool bat = bs.w != nullptr;
+    const char *nm_fxy = bat ? "batch_xy_fused_kernel" : "xy_fused_kernel";
     const char *nm_xy = bat ? "batch_f64_xymode" : "gemm_f64_xymode";
     const char *nm_x = bat ? "batch_f64_xmode" : "gemm_f64_xmode";
     const char *nm_y = bat ? "batch_f64_ymode" : "gemm_f64_ymode";
@@ -1075,6 +1322,22 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
         if (!banded && plan.streamed)  // up to the next t-point that can be streamed
             for (int e = 1; e < tc; ++e)
                 if (stream_run(m, t0 + e, t0 + e + 1, B, &tiles) > 0) tc = e;
+        if (plan.fused) {
+            // passes 1 and 2 in one: U_b((xo,yo),(zi,t)) straight from in_b
+            XYF f{};
+            f.in = in; f.fx = m.fx; f.fy = m.fy; f.U = U;
+            f.w = W; f.wS = wS;
+            f.nxi = (int)nxi; f.nyi = (int)nyi; f.nxo = (int)nxo; f.nyo = (int)nyo;
+            f.nzi = (int)nzi;
+            f.t0 = t0; f.tc = tc;
+            f.nin = nin; f.Ut = Ut;
+            f.xr = m.xr; f.yr = m.yr;
+            f.nxt = (int)((nxo + 15) / 16); f.nyt = (int)((nyo + 15) / 16);
+            f.gx = (int)((nxo + 63) / 64);
+            f.ldy = 16 * f.nyt;
+            f.remap = remap_default(8.0 * nxi * nyi * nzi);
+            DAGE_TRY(launch_xy(ctx, plan.fused, f, B, nm_fxy));
+        } else {
         // pass 1, batch (t, b): V_{b,t}((yi,zi), xo) = in_b((yi,zi), xi) . Fx_t^T(xi, xo)
         Gemm g1{};
         g1.A = in;
@@ -1127,6 +1390,7 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
         int nb2;
         set_tiles(g2, 1, (long)t0 * nyi, nyi, &nb2);
         DAGE_TRY(launch_gemm<1>(ctx, nm_y, g2, tc * B, nb2));
+        }
         }
 
         if (banded) {

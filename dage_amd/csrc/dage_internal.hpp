@@ -346,6 +346,9 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
                     const BatchSpec &bs, Workspace *ws);
 int apply_f64_batch_workspace(const ApplyMats &m, int B, size_t *bytes);
 int apply_f64_workspace(dage_operator op, size_t *bytes);
+// Allows the fused x/y pass its dynamic LDS on the current device (called
+// once per context, outside any stream capture).
+int prepare_fused_kernels();
 // Mixed-precision apply (apply_mixed.hip): npair = 6 (bf16x6) or 3 (bf16x3).
 int apply_mixed(dage_operator op, const double *in_dev, double *out_dev, int npair);
 // Batch of right-hand sides on one operator (same conventions as apply_f64_batch).

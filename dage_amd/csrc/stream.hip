@@ -541,12 +541,11 @@ int tile_ranges(const int *span, long row0, long n, long no, int2 *out) {
     return hb;
 }
 
-// Packed matrices and tables of the streamed passes; span: the row spans of
+// Ranges, packed matrices and tables of the streamed passes (axes up to 1024
+// points: the ranges only beyond); span: the row spans of
 // build_masks (x rows t*nxi.., then y, then z).
 int build_stream(dage_operator op, const std::vector<int> &span) {
     const long T = op->ntp;
-    for (int a = 0; a < 3; ++a)
-        if (op->din[a] > 1024 || op->dout[a] > 1024) return DAGE_OK;  // 64 tiles per mask
     long nt[3], nb[3], row[3], ranges = 0, r0 = 0;
     size_t pk = 0, off[3];
     for (int a = 0; a < 3; ++a) {
@@ -576,6 +575,15 @@ int build_stream(dage_operator op, const std::vector<int> &span) {
         }
         rp += T * nt[a];
     }
+    hipStream_t s = op->ctx->stream;
+    const size_t rb = sizeof(int2) * rg.size();
+    if (!op->d_ranges) DAGE_HIP_CHECK(hipMalloc((void **)&op->d_ranges, rb));
+    DAGE_HIP_CHECK(hipMemcpyAsync(op->d_ranges, rg.data(), rb, hipMemcpyHostToDevice, s));
+    for (int a = 0; a < 3; ++a)
+        if (op->din[a] > 1024 || op->dout[a] > 1024) {  // 64 tiles per mask
+            DAGE_HIP_CHECK(hipStreamSynchronize(s));
+            return DAGE_OK;
+        }
     // z steps: the panels of every t that some tile of the group needs, split
     // s of S taking the panels p of t with (t*nb + p) % S = s.  One list per
     // S: the split of the sum does not depend on which panels are skipped.
@@ -611,15 +619,11 @@ int build_stream(dage_operator op, const std::vector<int> &span) {
         op->z_t.resize(st.size());
         for (size_t i = 0; i < st.size(); ++i) op->z_t[i] = st[i].x;
     }
-    hipStream_t s = op->ctx->stream;
     if (!op->d_steps)  // every panel of every t, whatever the matrices hold
         DAGE_HIP_CHECK(hipMalloc((void **)&op->d_steps,
                                  sizeof(int4) * (size_t)(kMaxGroups * kMaxSplits * T * nb[2])));
     DAGE_HIP_CHECK(hipMemcpyAsync(op->d_steps, st.data(), sizeof(int4) * st.size(),
                                   hipMemcpyHostToDevice, s));
-    const size_t rb = sizeof(int2) * rg.size();
-    if (!op->d_ranges) DAGE_HIP_CHECK(hipMalloc((void **)&op->d_ranges, rb));
-    DAGE_HIP_CHECK(hipMemcpyAsync(op->d_ranges, rg.data(), rb, hipMemcpyHostToDevice, s));
     if (!op->d_pack) {
         DAGE_HIP_CHECK(hipMalloc((void **)&op->d_pack, 8 * pk));
         DAGE_TRY(fill_zero(op->ctx, op->d_pack, pk));
@@ -646,12 +650,10 @@ int build_stream(dage_operator op, const std::vector<int> &span) {
 }
 
 void stream_mats(dage_operator op, ApplyMats *m) {
-    if (!op->d_pack || !op->d_ranges) return;
-    const long T = op->ntp;
-    long nt[3];
-    for (int a = 0; a < 3; ++a) nt[a] = (op->dout[a] + 15) / 16;
+    if (!op->d_ranges) return;
     m->xr = op->d_ranges;
-    m->yr = m->xr + T * nt[0];
+    m->yr = m->xr + (long)op->ntp * ((op->dout[0] + 15) / 16);
+    if (!op->d_pack) return;
     m->fxp = op->d_pack + op->pack_off[0];
     m->fyp = op->d_pack + op->pack_off[1];
     m->fzp = op->d_pack + op->pack_off[2];
@@ -685,7 +687,7 @@ static char stream_mode() {
 
 // Whether the streamed passes take this operator's sizes at all.
 static bool streams(const ApplyMats &m) {
-    if (!m.xr || !m.fxp) return false;
+    if (!m.fxp) return false;
     // byte offsets within a plane of the cubes and 16 planes of U below 2^31
     if ((long)m.din[0] * (m.din[1] + 32) >= (1L << 28)) return false;
     if ((long)m.dout[0] * (m.dout[1] + 16) >= (1L << 24)) return false;

@@ -204,8 +204,9 @@ int dage_operator_apply_device_strided(dage_operator op, const double *in, int l
  * its intermediates in a fixed per-GPU scratch array of
  * dage_operator_noalloc_limit() bytes (128 MiB) that the library holds for
  * the life of the process.  The t-chunk shrinks to fit; when the
- * intermediates of one t-point (8*nxo*(nyi + nyo)*nzi bytes,
- * plus the z-pass partials) do not fit, DAGE_ERR_ARG is returned and nothing
+ * intermediates of one t-point (8*nxo*(nyi + nyo)*nzi bytes, with
+ * DAGE_APPLY_FUSED=1 and nxi and nyo up to 448 points 8*nxo*nyo*nzi, plus the
+ * z-pass partials) do not fit, DAGE_ERR_ARG is returned and nothing
  * is launched.  Calls no allocator.  Every call on one GPU shares that GPU's
  * array, so calls that overlap on one GPU (other streams, other contexts,
  * other host threads) race; calls on one stream are ordered. */

@@ -1,9 +1,11 @@
-"""The opt-in fused x/y pass (xy_fused_kernel, DAGE_APPLY_FUSED=1) against
-the separate x and y passes and the oracle.
+"""DAGE_APPLY_FUSED=1, the apply without the x pass's intermediate V in memory.
 
-With the same t-chunk (DAGE_APPLY_TCHUNK) both paths hand the z pass the same
-intermediate U, so their outputs must agree bit for bit; on its own chunking
-the fused path meets the FP64 bar, 1e-10 of max|V| against the oracle.
+Where every t-point can run on the streamed kernels those are used, else
+xy_fused_kernel (axes up to 448 points).  With the same t-chunk
+(DAGE_APPLY_TCHUNK) the fused kernel hands the z pass the same intermediate U
+as the separate passes, so without the streamed kernels
+(DAGE_APPLY_STREAM=0) their outputs must agree bit for bit; on its own
+chunking either way meets the FP64 bar, 1e-10 of max|V| against the oracle.
 """
 import os
 
@@ -73,20 +75,34 @@ def test_fused_equals_separate_passes(ctx, case):
         op.set_energy(energy)
         w = O.helmholtz_weights(q.tp, q.tw, energy)
     assert op.tiling()["band_t0"] == q.get_npoints() and op.tiling()["lowrank_t1"] == 0
-    fused = with_env({"DAGE_APPLY_TCHUNK": str(tchunk), "DAGE_APPLY_FUSED": "1"},
-                     lambda: op.transform_cube(rho))
-    sep = with_env({"DAGE_APPLY_TCHUNK": str(tchunk), "DAGE_APPLY_FUSED": "0"},
-                   lambda: op.transform_cube(rho))
+    def launched(env):
+        """The output and the launches of the fused, streamed and separate kernels."""
+        ctx.profile(True)
+        out = with_env(env, lambda: op.transform_cube(rho))
+        names = ("xy_fused_kernel", "gemm_f64_xymode", "gemm_f64_xmode")
+        ran = [ctx.profile_query(k)[1] > 0 for k in names]
+        ctx.profile(False)
+        return out, ran
+
+    same_u = {"DAGE_APPLY_TCHUNK": str(tchunk), "DAGE_APPLY_STREAM": "0"}
+    fused, ran = launched({**same_u, "DAGE_APPLY_FUSED": "1"})
+    assert ran == [True, False, False]
+    sep, ran = launched({**same_u, "DAGE_APPLY_FUSED": "0"})
+    assert ran == [False, False, True]
     ndiff = int(np.count_nonzero(fused != sep))
     print(f"case {case}: shape {fused.shape}, t-chunk {tchunk}: {ndiff} points differ")
     assert ndiff == 0
-    got = with_env({"DAGE_APPLY_FUSED": "1"}, lambda: op.transform_cube(rho))  # own t-chunking
+    own, ran = launched({"DAGE_APPLY_STREAM": "0", "DAGE_APPLY_FUSED": "1"})  # own t-chunking
+    assert ran == [True, False, False]
+    got, ran = launched({"DAGE_APPLY_FUSED": "1"})  # streamed: every axis is below 209 points
+    assert ran == [False, True, False]
     fx = O.exponentials(ain[0], aout[0], q.tp, False)
     fy = O.exponentials(ain[1], aout[1], q.tp, True)
     fz = O.exponentials(ain[2], aout[2], q.tp, True)
     coda = O.coda(q.tlog) if same else 0.0
     ref = O.transform_cube(fx, fy, fz, w, coda, rho, add_coda=same)
-    err = rel_maxdiff(got, ref)
-    print(f"case {case}: fused path vs oracle {err:.3e}")
-    assert err < 1e-10
+    for out in (own, got):
+        err = rel_maxdiff(out, ref)
+        print(f"case {case}: apply without V vs oracle {err:.3e}")
+        assert err < 1e-10
     op.close()

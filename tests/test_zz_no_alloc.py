@@ -102,3 +102,29 @@ def test_noalloc_apply_rejects_too_large(ctx):
     assert "workspace" in str(e.value)
     for obj in (a, b, op, g):
         obj.close()
+
+
+@pytest.mark.parametrize("shape", [(289, 161, 129), (161, 289, 129), (85, 85, 1029)])
+def test_noalloc_apply_without_v_on_long_axes(ctx, monkeypatch, shape):
+    """Boxes with an axis too long for the streamed kernels whose U and z
+    partial fit the scratch but not V beside them: refused, and accepted with
+    DAGE_APPLY_FUSED=1."""
+    g = dage_amd.Grid3D(ctx, [-0.1 * (n - 1) for n in shape], [np.full((n - 1) // 4, 0.8) for n in shape], 5)
+    q = dage_amd.GaussQuad(nlin=8, nlog=2, tlin=2.0, tlog=20.0)  # dense matrices at the first t
+    op = dage_amd.Coulomb3D(ctx, g, g, q)
+    limit = ctypes.c_size_t()
+    call("dage_operator_noalloc_limit", ctypes.byref(limit))
+    cube = 8 * np.prod(shape)
+    assert 2 * cube <= limit.value < 3 * cube
+    rho = np.asfortranarray(np.random.default_rng(5).uniform(-1.0, 1.0, shape))
+    a = dage_amd.DeviceCube(ctx, shape, rho)
+    b1, b2 = dage_amd.DeviceCube(ctx, shape), dage_amd.DeviceCube(ctx, shape)
+    with pytest.raises(DageError):
+        noalloc(op, a, b1)
+    monkeypatch.setenv("DAGE_APPLY_FUSED", "1")
+    noalloc(op, a, b1)
+    monkeypatch.delenv("DAGE_APPLY_FUSED")
+    device_apply(op, a, b2)
+    assert rel_maxdiff(b1.download(), b2.download()) < 1e-13
+    for obj in (a, b1, b2, op, g):
+        obj.close()

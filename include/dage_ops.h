@@ -518,8 +518,9 @@ int dage_batch_apply(dage_batch batch);
 /* The same work launched kernel by kernel (for profiling). */
 int dage_batch_apply_eager(dage_batch batch);
 /* Autotuner: times every GEMM column-block count 1..8 and the operator's own
- * tiling (0) for each pass of each grid group (reps timed runs each), keeps
- * the fastest and re-captures the graph.  tiles (optional, 3 per group)
+ * tiling (0) for each separate pass of each grid group (reps timed runs each),
+ * keeps the fastest and re-captures the graph; a group that runs no separate
+ * pass in FP64 keeps 0.  tiles (optional, 3 per group)
  * receives the choices.  Overwrites outputs. */
 int dage_batch_tune(dage_batch batch, int reps, int *tiles);
 int dage_batch_group_count(dage_batch batch, int *ngroups);

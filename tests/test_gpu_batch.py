@@ -161,3 +161,17 @@ def test_batch_slices_under_workspace_cap(ctx, monkeypatch, precision, tol):
         for i in range(len(sizes)):
             assert rel_maxdiff(sliced.download(i), ref[i]) < tol, i
     sliced.close()
+
+
+@pytest.mark.parametrize("stream", ["0", "1"])
+def test_tuning_of_fp64_groups(ctx, monkeypatch, stream):
+    """Column-block counts belong to the separate passes.  Where these run,
+    tuning replaces an operator's tiles of 128 columns on 33-point axes; where
+    every t-point runs streamed it has nothing to choose and reports the
+    operator's own."""
+    monkeypatch.setenv("DAGE_APPLY_STREAM", stream)
+    monkeypatch.setenv("DAGE_APPLY_NB", "8,8,8")
+    batch, *_ = make_batch(ctx, [33, 33, 33, 33], [-0.4, -1.5, -0.2, -3.0], seed=9)
+    tiles = batch.tune(reps=5)
+    print(tiles)
+    assert np.all(tiles == 0) if stream == "1" else np.all(tiles[:, :2] > 0)

@@ -192,11 +192,21 @@ def test_device_apply_and_chunking(ctx, monkeypatch):
     assert op2.workspace_bytes() < full
 
 
-def test_apply_block_sparse_matrices(ctx, monkeypatch):
+def separate_passes_ran(ctx):
+    """Whether the profiled applies ran the separate x pass, and not the streamed one."""
+    ran = ctx.profile_query("gemm_f64_xmode")[1] > 0, ctx.profile_query("gemm_f64_xymode")[1] > 0
+    ctx.profile(False)
+    return ran == (True, False)
+
+
+@pytest.mark.parametrize("stream", ["0", "1"])
+def test_apply_block_sparse_matrices(ctx, monkeypatch, stream):
     """Banded matrices with zeroed 16-row panels and an all-zero t: the GEMMs
     skip K panels that are zero on a block's columns.  A skipped panel adds
     exactly zero, so every column-block count gives bit-identical results,
-    and they match the oracle's dense apply."""
+    and they match the oracle's dense apply.  The streamed passes (stream 1),
+    which have no column blocks, match it too."""
+    monkeypatch.setenv("DAGE_APPLY_STREAM", stream)
     rng = np.random.default_rng(77)
     axes = [O.Axis.ncell_fixed(-4.0, 4.0, 5, 15), O.Axis.ncell_fixed(-3.0, 3.0, 5, 11),
             O.Axis.ncell_fixed(-5.0, 5.0, 5, 18)]
@@ -227,7 +237,9 @@ def test_apply_block_sparse_matrices(ctx, monkeypatch):
         monkeypatch.setenv("DAGE_APPLY_NB", nb)
         op = dage_amd.Coulomb3D(ctx, g, g, q, coda=False)
         op.set_matrices(fx, fy, fz)
+        ctx.profile(True)
         outs.append(op.transform_cube(cube))
+        assert separate_passes_ran(ctx) == (stream == "0")
         op.close()
     err = rel_maxdiff(outs[0], ref)
     print(f"block-sparse matrices vs oracle: {err:.3e}")
@@ -266,7 +278,9 @@ def test_apply_box_banded_matrices_pitch_tiles(ctx, monkeypatch):
     """Near-field style matrices: entry (i, j) is nonzero only when the boxes
     of 30 points holding i and j are neighbours.  The column tiles then follow
     the boxes (a pitch of 30 or 60, not a multiple of 16); the result is
-    bit-identical to 16-column tiles and matches the oracle."""
+    bit-identical to 16-column tiles and matches the oracle.  Tiles belong to
+    the separate passes."""
+    monkeypatch.setenv("DAGE_APPLY_STREAM", "0")
     rng = np.random.default_rng(78)
     ax = O.Axis.ncell_fixed(-4.0, 4.0, 7, 20)  # 121 points = 4 boxes of 30 (+1)
     n = ax.n
@@ -292,7 +306,9 @@ def test_apply_box_banded_matrices_pitch_tiles(ctx, monkeypatch):
     # x and y rows are one t each; the z pass's K runs over (zi, t), so its
     # panels straddle t and may not pay for a pitch
     assert all(p > 0 and p % 30 == 0 for p in tiling["pitch"][:2])
+    ctx.profile(True)
     got = op.transform_cube(cube)
+    assert separate_passes_ran(ctx)
     op.close()
     monkeypatch.setenv("DAGE_APPLY_NB", "2,2,2")
     op = dage_amd.Coulomb3D(ctx, g, g, q, coda=False)
@@ -306,13 +322,16 @@ def test_apply_box_banded_matrices_pitch_tiles(ctx, monkeypatch):
     assert np.array_equal(got, grid16)
 
 
-def test_direct_z_pass_accumulates_over_t_chunks(ctx, monkeypatch):
+@pytest.mark.parametrize("stream", ["0", "1"])
+def test_direct_z_pass_accumulates_over_t_chunks(ctx, monkeypatch, stream):
     """One right-hand side, no coda and a z pass without K split: the z pass
     accumulates every t-chunk straight into the output (no partials, no
     reduction).  A 1 MB workspace forces one t-point per chunk at 37^3 (40
     accumulating chunks, K = 37, so no split); the result matches the oracle
     and the split-K path (full workspace), with dense and with box-banded
-    (pitch-tiled) matrices."""
+    (pitch-tiled) matrices, for the separate z pass and the streamed one (two
+    t-points per chunk, in the space of V and U)."""
+    monkeypatch.setenv("DAGE_APPLY_STREAM", stream)
     rng = np.random.default_rng(91)
     ax = O.Axis.ncell_fixed(-6.0, 6.0, 7, 6)  # 37 points
     n = ax.n
@@ -342,7 +361,9 @@ def test_direct_z_pass_accumulates_over_t_chunks(ctx, monkeypatch):
         monkeypatch.setenv("DAGE_APPLY_WORKSPACE_MB", "1")
         op = dage_amd.Coulomb3D(ctx, g, g, q, coda=False)
         op.set_matrices(*mats)
+        ctx.profile(True)
         direct = op.transform_cube(cube)
+        assert separate_passes_ran(ctx) == (stream == "0")
         # V, U of one t-point and one unsplit z-pass partial (unused: the
         # z pass writes the output directly)
         assert op.workspace_bytes() == 3 * 8 * n ** 3 < full_ws
@@ -521,6 +542,7 @@ def test_t_grouped_x_pass_is_bit_identical(ctx, monkeypatch, n, energy):
     extra ones of the union over t add exact zeros) in the same order, so
     the apply is bit-identical; t-chunks of 3 and 4 (the last group of a
     chunk short)."""
+    monkeypatch.setenv("DAGE_APPLY_STREAM", "0")
     ax = O.Axis.ncell_fixed(-0.05 * (n - 1), 0.05 * (n - 1), 7, (n - 1) // 6)
     q = quad()
     g = lib_grid(ctx, [ax] * 3, 7)
@@ -537,7 +559,9 @@ def test_t_grouped_x_pass_is_bit_identical(ctx, monkeypatch, n, energy):
         res = {}
         for flag in ("1", "0"):
             monkeypatch.setenv("DAGE_APPLY_TGROUP", flag)
+            ctx.profile(True)
             res[flag] = op.transform_cube(cube)
+            assert separate_passes_ran(ctx)
         op.close()
         ndiff = int(np.count_nonzero(res["1"] != res["0"]))
         print(f"n {n}, t-chunk {tchunk}: t-grouped vs one-t x pass: {ndiff} points differ")

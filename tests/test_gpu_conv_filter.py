@@ -1,6 +1,6 @@
 """The filter gradient on FP32 MFMA (conv3d.hip) at the edges of its tiles:
-x segments and chunks (144 columns), row ranges that cross planes, every kind
-of channel count, against the FP64 oracle.
+x segments and chunks (144 columns), blocks of many rows whose ranges cross
+planes, every kind of channel count, against the FP64 oracle.
 
 A gradient is an FP32 sum of at most P = nx ny nz exact-product terms, added
 along chains of at most D terms (a lane group's 9 points of each of its
@@ -25,6 +25,10 @@ CASES = [
     (33, 7, 5, 3, 5), (64, 3, 3, 9, 16), (128, 2, 2, 16, 7),
     (1, 1, 1, 2, 16), (17, 9, 31, 2, 16), (129, 5, 3, 1, 16), (289, 2, 2, 2, 16),
     (17, 9, 31, 16, 1), (143, 3, 2, 16, 2), (145, 2, 2, 7, 1), (5, 4, 3, 1, 1), (600, 1, 2, 1, 1),
+    # several rows per block (1024 blocks with few channels, 256 with 16 x 16),
+    # the planes' rows no multiple of them: 5, 7, 9 and 5 rows, then 6 and 8
+    (5, 61, 83, 2, 16), (7, 83, 79, 1, 16), (6, 71, 127, 16, 1), (9, 67, 71, 16, 2),
+    (5, 37, 41, 16, 16), (18, 43, 47, 9, 16),
 ]
 
 

@@ -26,8 +26,8 @@ CASES = [
     ((47, 16, 33), None, 2, 0.3),
     ((8, 10, 12), (3, 5, 2), 5, 0.5),             # rectangular: always the full kernel
     ((24, 4, 10), (4, 24, 11), 4, 0.5),
-    ((16, 16, 16), None, 5, 0.6),                 # 65: rings of 3 beside the full 5
-    ((52, 22, 4), None, 5, 0.6),                  # 209 points: the widest full kernel is too small
+    ((16, 16, 16), None, 5, 0.6),                 # 65 points: five tiles, one launch
+    ((52, 22, 4), None, 5, 0.6),                  # 209 points: the full kernels are too small
 ]
 
 
@@ -150,3 +150,95 @@ def test_thin_boxes_keep_the_separate_passes(ctx, monkeypatch, shape, streams):
     op.transform_cuda_cube(a, b)
     assert rel_maxdiff(got, b.download()) < 1e-13
     op.close()
+
+
+def tile_kernels(ctx):
+    """The x/y kernels that the profiled applies launched."""
+    names = [f"stream_xy_{k}{n}" for k in ("full", "ring") for n in range(2, 14)]
+    ran = {k for k in names if ctx.profile_query(k)[1] > 0}
+    ctx.profile(False)
+    return ran
+
+
+# points per axis, band half-width in x and y (None: dense), t-points, the x/y
+# kernels
+KERNELS = [
+    ((17, 31, 5), None, 2, {"full2"}), ((33, 48, 5), None, 2, {"full3"}),
+    ((49, 64, 5), None, 2, {"full5"}), ((65, 80, 5), None, 2, {"full5"}),
+    ((96, 81, 5), None, 2, {"full6"}), ((97, 112, 5), None, 2, {"full7"}),
+    ((113, 17, 5), None, 2, {"full8"}), ((144, 129, 5), None, 2, {"full9"}),
+    ((145, 160, 5), None, 2, {"full10"}), ((161, 33, 5), None, 2, {"full11"}),
+    ((49, 177, 5), None, 2, {"full12"}), ((208, 193, 5), None, 2, {"full13"}),
+    ((81, 65, 5), 12, 2, {"ring3"}), ((129, 145, 5), 30, 2, {"ring5"}),
+    ((145, 143, 5), 48, 2, {"ring7"}), ((177, 161, 5), 64, 2, {"ring9"}),
+    ((193, 209, 5), 80, 2, {"ring11"}), ((225, 241, 5), 96, 2, {"ring13"}),
+    ((399, 33, 3), 96, 2, {"ring13"}), ((33, 399, 3), 96, 2, {"ring13"}),
+    # wide bands first, in launches of their own when each fills the card
+    ((225, 225, 65), (96,) * 3 + (12,) * 7, 10, {"ring13", "ring3"}),
+    # more than 13 z tiles (two groups), and more than 64 steps in a split
+    ((17, 17, 209), None, 3, {"full2"}), ((65, 65, 225), None, 40, {"full5"}),
+]
+
+
+@pytest.mark.parametrize("case", range(len(KERNELS)))
+def test_every_kernel(ctx, monkeypatch, case):
+    n, band, T, kernels = KERNELS[case]
+    q = dage_amd.GaussQuad(nlin=T, nlog=0, tlin=2.0, tlog=2.0)
+    rng = np.random.default_rng(case)
+
+    def matrix(axis):
+        m = n[axis]
+        F = rng.standard_normal((m, m, T))  # (out, in, t)
+        i = np.arange(m)
+        for t in range(T):
+            b = m if band is None or axis == 2 else band if np.isscalar(band) else band[t]
+            F[np.abs(i[:, None] - i) > b, t] = 0.0
+        return F
+
+    F = [matrix(a) for a in range(3)]
+    monkeypatch.setenv("DAGE_APPLY_STREAM", "1")
+    monkeypatch.setenv("DAGE_APPLY_BAND", "0")
+    g = dage_amd.Grid3D(ctx, [0.0] * 3, [np.full(m - 1, 0.2) for m in n], 2)
+    op = dage_amd.Coulomb3D(ctx, g, g, q, coda=False)
+    op.set_matrices(np.asfortranarray(F[0]), *(np.asfortranarray(F[a].transpose(1, 0, 2)) for a in (1, 2)))
+    x = rng.standard_normal(n)
+    w = O.coulomb_weights(q.tw)
+    ref, S = np.zeros(n), np.zeros(n)
+    for t in range(T):
+        v, s = x, np.abs(x)
+        for axis in range(3):
+            v = np.moveaxis(np.tensordot(F[axis][:, :, t], v, axes=(1, axis)), 0, axis)
+            s = np.moveaxis(np.tensordot(np.abs(F[axis][:, :, t]), s, axes=(1, axis)), 0, axis)
+        ref += w[t] * v
+        S += abs(w[t]) * s
+    a, b = dage_amd.DeviceCube(ctx, n, x), dage_amd.DeviceCube(ctx, n)
+    ctx.profile(True)
+    op.transform_cuda_cube(a, b)
+    assert tile_kernels(ctx) == {"stream_xy_" + k for k in kernels}
+    # the reference's own rounding has the same bound
+    err = np.abs(b.download() - ref) / (2 * (sum(n) + T + 3) * 2.0 ** -53 * S)
+    print(f"{n}: {err.max():.3f} of the bound")
+    assert np.all(err <= 1.0)
+    op.close()
+
+
+@pytest.mark.parametrize("n,energies", [(65, [-0.3, -1.1, -2.0]), (145, [-0.2, -0.9]), (33, [-0.5] * 7)])
+def test_batches(ctx, monkeypatch, n, energies):
+    """Right-hand sides with weights of their own, streamed and separate."""
+    g = dage_amd.Grid3D(ctx, [-0.05 * (n - 1)] * 3, [np.full((n - 1) // 4, 0.4)] * 3, 5)
+    q = dage_amd.GaussQuad(nlin=10, nlog=10, tlin=2.0, tlog=300.0)
+    rng = np.random.default_rng(n)
+    rhs = [rng.standard_normal((n, n, n)) for _ in energies]
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("DAGE_APPLY_STREAM", mode)
+        batch = dage_amd.HelmholtzBatch(ctx, [g] * len(rhs), energies, q)
+        for i, r in enumerate(rhs):
+            batch.upload(i, r)
+        ctx.profile(True)
+        batch.apply_eager()
+        assert bool(tile_kernels(ctx)) == (mode == "1")
+        got[mode] = [batch.download(i).copy() for i in range(len(rhs))]
+        batch.close()
+    for a, b in zip(got["0"], got["1"]):
+        assert rel_maxdiff(a, b) < 1e-13

@@ -115,6 +115,10 @@ void prof_end(dage_ctx ctx, const char *name, hipEvent_t start) {
     ctx->pending.push_back({start, stop, name});
 }
 
+void prof_count(dage_ctx ctx, const char *name) {
+    if (ctx->profiling) ctx->profile[name].launches += 1;
+}
+
 int prof_resolve(dage_ctx ctx) {
     if (ctx->pending.empty()) return DAGE_OK;
     DAGE_HIP_CHECK(hipStreamSynchronize(ctx->stream));

@@ -279,6 +279,8 @@ int ctx_scratch(dage_ctx ctx, size_t bytes, void **p);
 // Event-bracketed launch helpers (record only when profiling is on).
 void prof_begin(dage_ctx ctx, const char *name, hipEvent_t *start);
 void prof_end(dage_ctx ctx, const char *name, hipEvent_t start);
+// Counts a launch under a second name, without a time (no events).
+void prof_count(dage_ctx ctx, const char *name);
 int prof_resolve(dage_ctx ctx);
 
 // ----------------------------------------------------------------- kernels

@@ -812,12 +812,13 @@ int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, dou
     a.xr = m.xr; a.yr = m.yr;
     a.nxt = (a.nxo + 15) / 16; a.nyt = (a.nyo + 15) / 16;
     a.nxb = (a.nxi + 15) / 16; a.nyb = (a.nyi + 15) / 16;
-    // profiles count the launches of each kernel too
-    char kernel[32];
-    std::snprintf(kernel, sizeof kernel, "stream_xy_%s%d", tiles < 0 ? "full" : "ring", std::abs(tiles));
-    hipEvent_t ev, evk;
+    if (ctx->profiling) {
+        char kernel[32];
+        std::snprintf(kernel, sizeof kernel, "stream_xy_%s%d", tiles < 0 ? "full" : "ring", std::abs(tiles));
+        prof_count(ctx, kernel);
+    }
+    hipEvent_t ev;
     prof_begin(ctx, name, &ev);
-    prof_begin(ctx, kernel, &evk);
     int rc = DAGE_OK;
     hipStream_t s = ctx->stream;
     switch (tiles) {
@@ -840,7 +841,6 @@ int stream_xy(dage_ctx ctx, const ApplyMats &m, int tiles, const double *in, dou
     case -13: rc = launch_xy_n<13, false>(a, B, s); break;
     default: DAGE_REQUIRE(false, DAGE_ERR_STATE, "t-point %d is not streamed", t0);
     }
-    prof_end(ctx, kernel, evk);
     prof_end(ctx, name, ev);
     return rc;
 }

@@ -361,11 +361,11 @@ int launch_conv16(dage_ctx ctx, int nx, int ny, int nz, const float *in, const u
 //
 // Both replace a VALU kernel whose threads owned one (o, c) pair's 27 taps:
 // bound by its LDS reads (two per multiply-add of a tap) and, with few
-// channels, by idle threads.  129^3, 16 -> 16: 900 -> 314 us (29.7 GFLOP,
-// 195 us at the 152 TFLOP/s of a large FP32 product; the matrix cores are busy
-// 67 % of the time, the rest is the row barriers and the segments' padding
-// from 129 to 144 points); 2 -> 16: 900 -> 86, 16 -> 1: 900 -> 45 us (31 us for
-// the bytes at 4.7 TB/s).
+// channels, by idle threads.  Whole calls at 129^3, 16 -> 16: 1305 -> 328 us
+// (29.7 GFLOP, 195 us at the 152 TFLOP/s of a large FP32 product; the matrix
+// cores are busy 64 % of the time, the rest is the row barriers and the
+// segments' padding from 129 to 144 points); 2 -> 16: 630 -> 88, 16 -> 1: 1131 ->
+// 62 us (31 us for the bytes at 4.7 TB/s).
 constexpr int kSegL = 9;               // longest x segment of a lane group
 constexpr int kRowS = 16 * kSegL + 4;  // 148
 constexpr int kStage = 3;              // 64-float loads that cover a row
@@ -873,9 +873,11 @@ int dage_conv3d_backward_filter(dage_ctx ctx, int nx, int ny, int nz, int cin, i
     DAGE_TRY(use_device(ctx));
     DAGE_TRY(check_dims(nx, ny, nz, cin, cout));
     DAGE_REQUIRE(in && gout && gw && gb, DAGE_ERR_ARG, "bad argument");
-    const size_t smem = sizeof(float) * ((size_t)cin * 3 * (nx + 2) + (size_t)cout * nx);
-    DAGE_REQUIRE(smem <= 64 * 1024, DAGE_ERR_UNSUPPORTED, "x extent %d too long for one block",
-                 nx);
+    // The entry point's own limit: three rows of every input and one of every
+    // output channel in 64 KB (nx <= 254 at 16 x 16).  The kernels below cut x
+    // into chunks and would take any extent.
+    DAGE_REQUIRE(sizeof(float) * ((size_t)cin * 3 * (nx + 2) + (size_t)cout * nx) <= 64 * 1024,
+                 DAGE_ERR_UNSUPPORTED, "x extent %d beyond the 64 KB of rows", nx);
     // x chunks of at most 16*kSegL columns; blocks of rows for one block per
     // CU (16 x 16 channels: 132 KB of LDS) or four (the few-channel kernel,
     // bound by its loads)

@@ -215,8 +215,9 @@ int dage_operator_apply_device_noalloc(dage_operator op, const double *cubein_de
 int dage_operator_noalloc_limit(size_t *bytes);
 /* Bytes of device workspace the operator holds for its intermediates. */
 int dage_operator_workspace_bytes(dage_operator op, size_t *bytes);
-/* No reference counterpart (diagnostic): the output-column tiling the FP64
- * passes x, y, z use, chosen from the matrices' zero blocks.  nb[p]: 16-wide
+/* No reference counterpart (diagnostic): the output-column tiling of the
+ * separate FP64 passes x, y, z (those that run where the streamed passes do
+ * not), chosen from the matrices' zero blocks.  nb[p]: 16-wide
  * column blocks per tile (0: picked from the output width at each apply);
  * pitch[p]: tile pitch in points, 0 for tiles of 16*nb[p] columns;
  * skip[p]: 1 when all-zero K panels are skipped. */
@@ -578,7 +579,8 @@ int dage_conv3d_forward(dage_ctx ctx, int nx, int ny, int nz, int cin, int cout,
 int dage_conv3d_backward_data(dage_ctx ctx, int nx, int ny, int nz, int cin,
                               int cout, const float *grad_out,
                               const unsigned short *w_bf16, float *grad_in);
-/* Deterministic filter and bias gradients (fixed-order two-stage sums). */
+/* Deterministic filter and bias gradients (fixed-order two-stage sums).
+ * 4*(3*cin*(nx + 2) + cout*nx) must not exceed 65536 (DAGE_ERR_UNSUPPORTED). */
 int dage_conv3d_backward_filter(dage_ctx ctx, int nx, int ny, int nz, int cin,
                                 int cout, const float *in, const float *grad_out,
                                 float *grad_w, float *grad_b);

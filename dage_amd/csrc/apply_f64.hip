@@ -1221,10 +1221,14 @@ int apply_f64_batch(dage_ctx ctx, const ApplyMats &m, const double *in, double *
     const long nxi = m.din[0], nyi = m.din[1], nzi = m.din[2];
     const long nxo = m.dout[0], nyo = m.dout[1], nzo = m.dout[2];
     const int T = m.ntp, B = bs.B;
-    const Plan plan = make_plan(m, B, bs.ws_cap);
+    Plan plan = make_plan(m, B, bs.ws_cap);
+    // a reserved workspace holds the plan of its reservation; a route chosen
+    // since then (DAGE_APPLY_STREAM) makes do with it
+    if (bs.no_alloc && 8 * (plan.v_elems + plan.u_elems + plan.p_elems) > ws->bytes)
+        plan = make_plan(m, B, ws->bytes);
     DAGE_REQUIRE(plan.tchunk > 0, DAGE_ERR_ARG,
                  "the apply needs more than the %zu bytes of workspace it may use (the "
-                 "intermediates of one t-point do not fit)", bs.ws_cap);
+                 "intermediates of one t-point do not fit)", ws->bytes);
     const size_t need = 8 * (plan.v_elems + plan.u_elems + plan.p_elems);
     if (need > ws->bytes) {
         DAGE_REQUIRE(!bs.no_alloc, DAGE_ERR_STATE, "workspace of %zu bytes not reserved", need);

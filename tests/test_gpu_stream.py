@@ -239,6 +239,11 @@ def test_batches(ctx, monkeypatch, n, energies):
         batch.apply_eager()
         assert bool(tile_kernels(ctx)) == (mode == "1")
         got[mode] = [batch.download(i).copy() for i in range(len(rhs))]
+        # the other route in the workspace that was reserved for this one
+        monkeypatch.setenv("DAGE_APPLY_STREAM", "1" if mode == "0" else "0")
+        batch.apply_eager()
+        for i in range(len(rhs)):
+            assert rel_maxdiff(batch.download(i), got[mode][i]) < 1e-13
         batch.close()
     for a, b in zip(got["0"], got["1"]):
         assert rel_maxdiff(a, b) < 1e-13

@@ -361,7 +361,7 @@ int launch_conv16(dage_ctx ctx, int nx, int ny, int nz, const float *in, const u
 //
 // Both replace a VALU kernel whose threads owned one (o, c) pair's 27 taps:
 // bound by its LDS reads (two per multiply-add of a tap) and, with few
-// channels, by idle threads.  Whole calls at 129^3, 16 -> 16: 1305 -> 328 us
+// channels, by idle threads.  Whole calls at 129^3, 16 -> 16: 1305 -> 310 us
 // (29.7 GFLOP, 195 us at the 152 TFLOP/s of a large FP32 product; the matrix
 // cores are busy 64 % of the time, the rest is the row barriers and the
 // segments' padding from 129 to 144 points); 2 -> 16: 630 -> 88, 16 -> 1: 1131 ->
@@ -406,6 +406,7 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
     const long r0 = (long)blockIdx.x * rows_per_block;
     const long r1 = min(nrows, r0 + rows_per_block);
     const int start = (4 * w + k) * L, last = nx - x0 - start;
+    const bool padded = nx - x0 < 4 * (w + 1) * L && nx - x0 >= 4 * w * L;  // holds column nx
 
     // A row's sums start at zero and are added to the block's after it: chains
     // of L matrix products and of the rows instead of their product (one
@@ -460,6 +461,43 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
         }
     };
 
+    // One row's products.  The left tap of the first padding column is
+    // in[nx - 1], times a zero of gout: where that is not finite, MASK makes it
+    // zero (in every row, 129^3 at 16 x 16: 328 us instead of 310).
+    auto add_row = [&](int y, auto mask) {
+        constexpr bool MASK = decltype(mask)::value;
+        const float *go = sm + (12 + (y & 1)) * ROW + n * kRowS + start;
+        const float *ir[3];
+        float v0[3], v1[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            ir[d] = sm + (4 * dz + ((y + d - 1) & 3)) * ROW + n * kRowS + start;
+            v0[d] = !MASK || 0 < last ? ir[d][0] : 0.0f;
+            v1[d] = ir[d][1];
+        }
+        f4 acc[9];
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+        float accb = 0.0f;
+#pragma unroll
+        for (int x = 0; x < L; ++x) {
+            const float g = go[x];
+            accb += g;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const float v2 = ir[d][x + 2];
+                acc[3 * d] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v0[d], acc[3 * d], 0, 0, 0);
+                acc[3 * d + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v1[d], acc[3 * d + 1], 0, 0, 0);
+                acc[3 * d + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v2, acc[3 * d + 2], 0, 0, 0);
+                v0[d] = !MASK || x + 1 < last ? v1[d] : 0.0f;
+                v1[d] = v2;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 9; ++t) sum[t] += acc[t];
+        sumb += accb;
+    };
+
     for (long row = r0; row < r1;) {
         const int z = (int)(row / ny), ya = (int)(row - (long)z * ny);
         const int yb = (int)min((long)ny, ya + r1 - row);  // rows [ya, yb) of plane z
@@ -474,38 +512,13 @@ __global__ void __launch_bounds__(768) conv_filter_mfma_kernel(const float *in, 
             // row y + 2 replaces y - 2, output row y + 1 replaces y - 1
             load_in(y + 2, z);
             load_out(y + 1, z);
-            const float *go = sm + (12 + (y & 1)) * ROW + n * kRowS + start;
-            const float *ir[3];
-            float v0[3], v1[3];
+            bool bad = false;
+            if (padded)
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                ir[d] = sm + (4 * dz + ((y + d - 1) & 3)) * ROW + n * kRowS + start;
-                // the left tap of the first padding column is in[nx - 1]; as
-                // zero it cannot turn an infinity there into a NaN
-                v0[d] = 0 < last ? ir[d][0] : 0.0f;
-                v1[d] = ir[d][1];
-            }
-            f4 acc[9];
-#pragma unroll
-            for (int t = 0; t < 9; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-            float accb = 0.0f;
-#pragma unroll
-            for (int x = 0; x < L; ++x) {
-                const float g = go[x];
-                accb += g;
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    const float v2 = ir[d][x + 2];
-                    acc[3 * d] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v0[d], acc[3 * d], 0, 0, 0);
-                    acc[3 * d + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v1[d], acc[3 * d + 1], 0, 0, 0);
-                    acc[3 * d + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, v2, acc[3 * d + 2], 0, 0, 0);
-                    v0[d] = x + 1 < last ? v1[d] : 0.0f;
-                    v1[d] = v2;
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < 9; ++t) sum[t] += acc[t];
-            sumb += accb;
+                for (int d = 0; d < 3; ++d)
+                    bad |= !__builtin_isfinite(sm[(4 * dz + ((y + d - 1) & 3)) * ROW + n * kRowS + nx - x0]);
+            if (__builtin_expect(__any(bad), 0)) add_row(y, std::true_type{});
+            else add_row(y, std::false_type{});
             store_in(y + 2);
             store_out(y + 1);
             __syncthreads();

@@ -363,7 +363,7 @@ int launch_conv16(dage_ctx ctx, int nx, int ny, int nz, const float *in, const u
 // bound by its LDS reads (two per multiply-add of a tap) and, with few
 // channels, by idle threads.  Whole calls at 129^3, 16 -> 16: 1305 -> 310 us
 // (29.7 GFLOP, 195 us at the 152 TFLOP/s of a large FP32 product; the matrix
-// cores are busy 64 % of the time, the rest is the row barriers and the
+// cores are busy 67 % of the time, the rest is the row barriers and the
 // segments' padding from 129 to 144 points); 2 -> 16: 630 -> 88, 16 -> 1: 1131 ->
 // 62 us (31 us for the bytes at 4.7 TB/s).
 constexpr int kSegL = 9;               // longest x segment of a lane group

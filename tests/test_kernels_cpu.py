@@ -3,10 +3,11 @@ compiler writes for each one into the gfx950 code objects."""
 import os
 import struct
 
-import msgpack
 import pytest
 
 import dage_amd._lib as lib
+
+msgpack = pytest.importorskip("msgpack")
 
 SO = os.path.join(os.path.dirname(lib.__file__), "libdage_ops.so")
 NT_AMDGPU_METADATA = 32
